@@ -56,8 +56,7 @@ static layer_geo dec_geo(int i) {
 
 struct ptd_model {
   void *slab;                      /* relaid weights, biases, tail constants */
-  const float *wr[PTD_DEC_NLAYER]; /* MFMA layout [Mp/32][K][cinp/8][64][4] */
-  const float *wr16[PTD_DEC_NLAYER]; /* for 16-row tiles [Mp/16][K][cinp/8][64][2] */
+  const float *wr[PTD_DEC_NLAYER]; /* MFMA layout (ptk_relayout) */
   const float *b[PTD_DEC_NLAYER];
   const float *consts;             /* the tail's table: hann, basis_c, basis_s, final conv */
   layer_geo g[PTD_DEC_NLAYER];
@@ -117,7 +116,7 @@ ptd_model *ptdi_model_build(pt_ctx *c, const void *const *w, const int *wisz, co
   ptd_model *m = calloc(1, sizeof *m);
   if (!m) return NULL;
   size_t total = 0, packed_max = 0, half_max = 0;
-  size_t off_w[PTD_DEC_NLAYER], off_w16[PTD_DEC_NLAYER], off_b[PTD_DEC_NLAYER];
+  size_t off_w[PTD_DEC_NLAYER], off_b[PTD_DEC_NLAYER];
   int64_t wn[PTD_DEC_NLAYER];
   const int last = PTD_DEC_NLAYER - 1;
   if (!w[last] || (wisz && wisz[last] != 4)) {
@@ -141,8 +140,6 @@ ptd_model *ptdi_model_build(pt_ctx *c, const void *const *w, const int *wisz, co
     if (isz == 2 && (size_t) wn[i] * 2 > half_max) half_max = (size_t) wn[i] * 2;
     off_w[i] = total;
     total += al256(ptk_relayout_floats(M, K, g.cin) * sizeof(float));
-    off_w16[i] = total;
-    total += al256(ptk_relayout16_floats(M, K, g.cin) * sizeof(float));
     off_b[i] = total;
     total += al256((size_t) g.cout * sizeof(float));
   }
@@ -172,12 +169,10 @@ ptd_model *ptdi_model_build(pt_ctx *c, const void *const *w, const int *wisz, co
      * column's four phases as consecutive samples */
     const int il = g.convT ? M / 4 : 0;
     if (up || ptk_relayout_il((float *) (base + off_w[i]), tmp, M, K, g.cin, il, c->g_stream) ||
-        ptk_relayout16_il((float *) (base + off_w16[i]), tmp, M, K, g.cin, il, c->g_stream) ||
         ptk_h2d_async(base + off_b[i], b[i], (size_t) g.cout * sizeof(float), c->g_stream) ||
         ptk_stream_sync(c->g_stream))
       goto fail;
     m->wr[i] = (const float *) (base + off_w[i]);
-    m->wr16[i] = (const float *) (base + off_w16[i]);
     m->b[i] = (const float *) (base + off_b[i]);
   }
   if (ptk_h2d_async(base + off_c, consts, sizeof consts, c->g_stream) || ptk_stream_sync(c->g_stream))
@@ -213,7 +208,6 @@ static void conv_layer_desc(ptk_conv_desc *d, const ptd_model *m, int i, const f
   const int c4 = (g.cout + 3) / 4 * 4;
   ptdi_conv_desc(d, x, ldx, (int64_t) g.cin * ldx, T, g.cin, m->wr[i], m->b[i], g.cout, g.K, 1,
                  g.sd, g.pad, c4, y, ldy, (int64_t) c4 * ldy, T, batch);
-  d->w16 = m->wr16[i];
 }
 
 static void epi_push(ptk_conv_desc *d, int op, float a, const float *t, int64_t ldt, int64_t bst) {
@@ -447,26 +441,50 @@ int ptd_window_cols(int64_t T, int batch, int64_t lo_first, int64_t lo, int64_t 
   return on;
 }
 
-/* One MRF depth for `batch` items: c1 group then c2 group (see ptd_mrf_depth).  xinL[br]: the
- * LeakyReLU(0.1)'d input of branch br, or NULL to apply the LeakyReLU while staging xin[br];
- * yL: when not NULL, c2 also writes LeakyReLU(0.1) of its output there. */
-static int mrf_depth(pt_ctx *c, const ptd_model *m, int stage, int j, const float *const *xin,
-                     const float *const *xinL, float *const *a, float *const *y,
-                     float *const *yL, int64_t T, int batch, const cols_t (*cols)[2]) {
+/* d reads split planes: LeakyReLU(in_a) of its x */
+static void in_split(ptk_conv_desc *d, const void *xsp, float in_a) {
+  d->in_op = PTK_IN_SPLIT;
+  d->xsp = xsp;
+  d->in_a = in_a;
+}
+
+/* One MRF depth for `batch` items: c1 group then c2 group (see ptd_mrf_depth).  The c1 input,
+ * LeakyReLU(0.1)(xin[br]): as split planes in xinS[br], or as fp32 in xinL[br], or neither (applied
+ * to xin[br] as it is staged).  aS: when not NULL, c1 also writes its output as split planes there
+ * and c2 reads them.  yL / yS: when not NULL, c2 also writes LeakyReLU(0.1) of its output there, as
+ * fp32 / as split planes. */
+typedef struct {
+  const float *const *xin, *const *xinL;
+  const void *const *xinS;
+  float *const *a;
+  void *const *aS;
+  float *const *y, *const *yL;
+  void *const *yS;
+} depth_io;
+static int mrf_depth(pt_ctx *c, const ptd_model *m, int stage, int j, const depth_io *io, int64_t T,
+                     int batch, const cols_t (*cols)[2]) {
   const int base = stage == 0 ? 2 : 21, C = stage == 0 ? 256 : 128;
   ptk_conv_desc d1[3], d2[3];
   for (int br = 0; br < 3; br++) {
     const int i1 = base + br * 6 + j * 2, i2 = i1 + 1;
-    conv_layer_desc(&d1[br], m, i1, xinL ? xinL[br] : xin[br], T, T, batch, a[br], T);
-    if (!xinL) {
+    conv_layer_desc(&d1[br], m, i1, io->xinL ? io->xinL[br] : io->xin[br], T, T, batch, io->a[br], T);
+    if (io->xinS) {
+      in_split(&d1[br], io->xinS[br], 0.1f);
+    } else if (!io->xinL) {
       d1[br].in_op = PTK_IN_LEAKY;
       d1[br].in_a = 0.1f;
     }
     epi_push(&d1[br], PTK_EPI_LEAKY, 0.1f, NULL, 0, 0);
-    conv_layer_desc(&d2[br], m, i2, a[br], T, T, batch, y[br], T);
-    epi_push(&d2[br], PTK_EPI_ADDT, 0.0f, xin[br], T, (int64_t) C * T);
-    if (yL) {
-      d2[br].y2 = yL[br];
+    conv_layer_desc(&d2[br], m, i2, io->a[br], T, T, batch, io->y[br], T);
+    if (io->aS) {
+      d1[br].ysp = io->aS[br];
+      d1[br].a2 = 1.0f;
+      in_split(&d2[br], io->aS[br], 1.0f);
+    }
+    epi_push(&d2[br], PTK_EPI_ADDT, 0.0f, io->xin[br], T, (int64_t) C * T);
+    if (io->yL || io->yS) {
+      d2[br].y2 = io->yL ? io->yL[br] : NULL;
+      d2[br].ysp = io->yS ? io->yS[br] : NULL;
       d2[br].a2 = 0.1f;
     }
     if (cols) {
@@ -486,35 +504,47 @@ int ptd_mrf_depth(pt_ctx *c, const ptd_model *m, int stage, int depth, const flo
                   float *const *y_leaky, int64_t T) {
   if (!c || !c->use_cuda || !m || (stage != 0 && stage != 1) || depth < 0 || depth > 2 || T < 1)
     return -1;
-  return mrf_depth(c, m, stage, depth, xin, xin_leaky, a, y, y_leaky, T, 1, NULL);
+  /* c2's input as split planes, when the arena has room for them */
+  const size_t tb = (size_t) (stage == 0 ? 256 : 128) * T * sizeof(float);
+  void *mark = ptdi_arena_mark(c);
+  void *aS[3] = {ptdi_arena_alloc(c, tb), ptdi_arena_alloc(c, tb), ptdi_arena_alloc(c, tb)};
+  const depth_io io = {.xin = xin, .xinL = xin_leaky, .a = a, .aS = aS[0] && aS[1] && aS[2] ? aS : NULL,
+                       .y = y, .yL = y_leaky};
+  const int rc = mrf_depth(c, m, stage, depth, &io, T, 1, NULL);
+  ptdi_arena_release(c, mark);
+  return rc;
 }
 
-/* MRF stack on x [batch][C][T] (xL = LeakyReLU(0.1)(x), or NULL): writes the three branch
- * outputs (before the average) */
-static int mrf_run(pt_ctx *c, const ptd_model *m, int stage, const float *x, const float *xL,
+/* MRF stack on x [batch][C][T] (xS: LeakyReLU(0.1)(x) as split planes, or NULL): writes the three
+ * branch outputs (before the average) */
+static int mrf_run(pt_ctx *c, const ptd_model *m, int stage, const float *x, const void *xS,
                    int64_t T, int batch, float *const out[3], const cone_plan *cp) {
   const cols_t(*cols)[3][2] = cp ? cp->mrf[stage] : NULL;
   const int C = stage == 0 ? 256 : 128;
   const size_t tb = (size_t) batch * C * T * sizeof(float);
-  float *a[3], *yb[3], *lb[3];
+  float *a[3];
+  void *aS[3], *yS[3];
   for (int br = 0; br < 3; br++) {
     a[br] = ptdi_arena_alloc(c, tb);
-    yb[br] = ptdi_arena_alloc(c, tb);
-    lb[br] = ptdi_arena_alloc(c, tb);
-    if (!a[br] || !yb[br] || !lb[br]) {
+    aS[br] = ptdi_arena_alloc(c, tb);
+    yS[br] = ptdi_arena_alloc(c, tb);
+    if (!a[br] || !aS[br] || !yS[br]) {
       PT_LOG("arena too small for the MRF stack (T %lld batch %d)", (long long) T, batch);
       return -1;
     }
   }
-  /* depth 0: x -> out[] (+ lb[]); depth 1: out[] -> yb[] (+ lb[], rewritten after depth 1's c1
-   * has read it: same stream); depth 2: yb[] -> out[] */
-  const float *xs[3] = {x, x, x}, *xls[3] = {xL, xL, xL};
-  if (mrf_depth(c, m, stage, 0, xs, xL ? xls : NULL, a, out, lb, T, batch, cols ? cols[0] : NULL))
-    return -1;
-  const float *p1[3] = {out[0], out[1], out[2]}, *l1[3] = {lb[0], lb[1], lb[2]};
-  if (mrf_depth(c, m, stage, 1, p1, l1, a, yb, lb, T, batch, cols ? cols[1] : NULL)) return -1;
-  const float *p2[3] = {yb[0], yb[1], yb[2]};
-  return mrf_depth(c, m, stage, 2, p2, l1, a, out, NULL, T, batch, cols ? cols[2] : NULL);
+  /* depth 0: x -> out[]; depths 1 and 2: out[] in place (a c2 reads the residual it overwrites in
+   * the lane that writes it).  yS[] is rewritten by a depth's c2 after its c1 has read it. */
+  const float *xs[3] = {x, x, x}, *os[3] = {out[0], out[1], out[2]};
+  const void *xSs[3] = {xS, xS, xS}, *ySs[3] = {yS[0], yS[1], yS[2]};
+  depth_io io = {.xin = xs, .xinS = xS ? xSs : NULL, .a = a, .aS = aS, .y = out, .yS = yS};
+  for (int j = 0; j < 3; j++) {
+    if (j == 2) io.yS = NULL;
+    if (mrf_depth(c, m, stage, j, &io, T, batch, cols ? cols[j] : NULL)) return -1;
+    io.xin = os;
+    io.xinS = ySs;
+  }
+  return 0;
 }
 
 int ptd_tail(pt_ctx *c, const ptd_model *m, const float *p, int64_t L, int batch, float *wav) {
@@ -560,58 +590,65 @@ static int decode_impl(pt_ctx *c, const ptd_model *m, const float *z, int64_t ld
   if (emit && !stages && cone_enabled() && cone_plan_make(&plan, T, batch, emit) == 0) cp = &plan;
   void *mark = ptdi_arena_mark(c);
   int rc = -1;
+  /* S: the LeakyReLU'd copy a conv reads, as split planes (the same bytes as the fp32 tensor) */
   float *h = ptdi_arena_alloc(c, f * 512 * T);
+  void *hS = ptdi_arena_alloc(c, f * 512 * T);
   float *x0 = ptdi_arena_alloc(c, f * 256 * T1);
-  float *x0L = ptdi_arena_alloc(c, f * 256 * T1);
+  void *x0S = ptdi_arena_alloc(c, f * 256 * T1);
   float *o0[3] = {ptdi_arena_alloc(c, f * 256 * T1), ptdi_arena_alloc(c, f * 256 * T1),
                   ptdi_arena_alloc(c, f * 256 * T1)};
-  if (!h || !x0 || !x0L || !o0[0] || !o0[1] || !o0[2]) goto oom;
+  if (!h || !hS || !x0 || !x0S || !o0[0] || !o0[1] || !o0[2]) goto oom;
   ptk_conv_desc d;
   /* conv_pre + LeakyReLU */
   ptdi_conv_desc(&d, z, ldz, bsz, T, 192, m->wr[0], m->b[0], 512, 7, 1, 1, 3, 512, h, T, 512 * T, T,
                  batch);
-  d.w16 = m->wr16[0];
   epi_push(&d, PTK_EPI_LEAKY, 0.1f, NULL, 0, 0);
+  d.ysp = hS;
+  d.a2 = 1.0f;
   if (cp) cols_apply(&d, &cp->pre);
   if (ptk_conv_launch(&d, 1, c->g_stream)) goto fail;
   /* ups.0 */
   ptdi_convT_desc(&d, h, T, 512 * T, T, 512, m->wr[1], m->b[1], 256, 4, 6, 16, x0, T1, 256 * T1, batch);
-  d.w16 = m->wr16[1];
+  in_split(&d, hS, 1.0f);
   d.phase_il = 1;
-  d.y2 = x0L;
+  d.ysp = x0S;
   d.a2 = 0.1f;
   if (cp) cols_apply(&d, &cp->up0);
   if (ptk_conv_launch(&d, 1, c->g_stream)) goto fail;
   void *mark1 = ptdi_arena_mark(c);
-  if (mrf_run(c, m, 0, x0, x0L, T1, batch, o0, cp)) goto fail;
+  if (mrf_run(c, m, 0, x0, x0S, T1, batch, o0, cp)) goto fail;
   ptdi_arena_release(c, mark1);   /* the MRF temporaries; o0[] stay */
   float *x1 = ptdi_arena_alloc(c, f * 128 * T2);
-  float *x1L = ptdi_arena_alloc(c, f * 128 * T2);
+  void *x1S = ptdi_arena_alloc(c, f * 128 * T2);
   float *o1[3] = {ptdi_arena_alloc(c, f * 128 * T2), ptdi_arena_alloc(c, f * 128 * T2),
                   ptdi_arena_alloc(c, f * 128 * T2)};
-  if (!x1 || !x1L || !o1[0] || !o1[1] || !o1[2]) goto oom;
+  if (!x1 || !x1S || !o1[0] || !o1[1] || !o1[2]) goto oom;
+  void *mark2 = ptdi_arena_mark(c);
   /* ups.1 over leaky(avg(branches), 0.1) */
   float *av0 = ptdi_arena_alloc(c, f * 256 * T1);
-  if (!av0 || ptk_avg3_leaky(o0[0], o0[1], o0[2], av0, (int64_t) batch * 256 * T1, 0.1f, c->g_stream)) goto fail;
+  void *av0S = ptdi_arena_alloc(c, f * 256 * T1);
+  if (!av0 || !av0S) goto oom;
+  if (ptk_avg3_leaky_split(o0[0], o0[1], o0[2], av0, av0S, (int64_t) batch * 256, T1, 0.1f, c->g_stream)) goto fail;
   ptdi_convT_desc(&d, av0, T1, 256 * T1, T1, 256, m->wr[20], m->b[20], 128, 4, 6, 16, x1, T2,
                   128 * T2, batch);
-  d.w16 = m->wr16[20];
+  in_split(&d, av0S, 1.0f);
   d.phase_il = 1;
-  d.y2 = x1L;
+  d.ysp = x1S;
   d.a2 = 0.1f;
   if (cp) cols_apply(&d, &cp->up1);
   if (ptk_conv_launch(&d, 1, c->g_stream)) goto fail;
-  void *mark2 = ptdi_arena_mark(c);
-  if (mrf_run(c, m, 1, x1, x1L, T2, batch, o1, cp)) goto fail;
+  ptdi_arena_release(c, mark2);
+  if (mrf_run(c, m, 1, x1, x1S, T2, batch, o1, cp)) goto fail;
   ptdi_arena_release(c, mark2);
   float *p = ptdi_arena_alloc(c, f * 72 * L);
-  if (!p) goto oom;
   /* conv_post over reflect_pad(1,0)(leaky(avg(branches), 0.01)) */
   float *av1 = ptdi_arena_alloc(c, f * 128 * T2);
-  if (!av1 || ptk_avg3_leaky(o1[0], o1[1], o1[2], av1, (int64_t) batch * 128 * T2, 0.01f, c->g_stream)) goto fail;
+  void *av1S = ptdi_arena_alloc(c, f * 128 * T2);
+  if (!p || !av1 || !av1S) goto oom;
+  if (ptk_avg3_leaky_split(o1[0], o1[1], o1[2], av1, av1S, (int64_t) batch * 128, T2, 0.01f, c->g_stream)) goto fail;
   ptdi_conv_desc(&d, av1, T2, 128 * T2, L, 128, m->wr[39], m->b[39], 72, 7, 1, 1, 3, 72, p, L,
                  72 * L, L, batch);
-  d.w16 = m->wr16[39];
+  in_split(&d, av1S, 1.0f);
   d.reflect_l1 = 1;
   if (cp) cols_apply(&d, &cp->post);
   if (ptk_conv_launch(&d, 1, c->g_stream)) goto fail;
@@ -705,7 +742,6 @@ static int layer_run(pt_ctx *c, const ptd_model *m, int layer, const float *x, i
     const int64_t Lout = (T - 1) * g.sd - 2 * g.pad + g.K;
     ptdi_convT_desc(&d, x, T, (int64_t) g.cin * T, T, g.cin, m->wr[layer], m->b[layer], g.cout,
                     g.sd, g.pad, g.K, y, Lout, (int64_t) c4 * Lout, batch);
-    d.w16 = m->wr16[layer];
     d.phase_il = 1;
   } else {
     conv_layer_desc(&d, m, layer, x, T, T, batch, y, T);

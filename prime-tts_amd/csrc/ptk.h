@@ -73,7 +73,9 @@ void ptk_knobs_reload(void);
  * c outside [0, lim) reads 0 (in-kernel zero padding and the convT tail flush).
  * Output for row m = r*C4 + co and column q goes to  y[b*bsy + co*ldy + (q*ys + r - ypad)]
  * when that index is in [0, Lout) (conv: C4 = M, ys = 1, ypad = 0). */
-enum { PTK_IN_PLAIN = 0, PTK_IN_LEAKY = 1 };
+/* input transform: none, LeakyReLU(in_a) as x is read, or LeakyReLU(in_a) of x already in split
+   planes (xsp) */
+enum { PTK_IN_PLAIN = 0, PTK_IN_LEAKY = 1, PTK_IN_SPLIT = 2 };
 enum {
   PTK_EPI_NONE = 0,
   PTK_EPI_LEAKY = 1,   /* v >= 0 ? v : a*v                        (reference op code 1) */
@@ -101,21 +103,22 @@ typedef struct {
   int cin;
   int in_op;
   float in_a;
+  /* PTK_IN_SPLIT: LeakyReLU(in_a) of x as split planes [cin/8][2][ldx][8] (see ptk_kernels.hip),
+     batch stride bsx floats; x itself is read only for columns whose magnitudes the planes do not
+     hold.  cin a multiple of 16, 16-byte aligned. */
+  const void *xsp;
   int reflect_l1;             /* virtual column 0 reads physical column 1, column c>0 reads c-1 */
-  /* weights: relaid [Mp/32][K][cinp/8][64][4] (see ptk_relayout) */
+  /* weights: relaid (see ptk_relayout) */
   const float *w;
-  /* optional: the same weights relaid for 16-row tiles [Mp/16][K][cinp/8][64][2]
-     (ptk_relayout16); NULL keeps the launch on 32-row tiles */
-  const float *w16;
   int cinp;
   const float *bias;
   int nbias;
   int K, dil, stride, shift;
   int M;                      /* GEMM rows (cout4 or s*cout4) */
   int C4;                     /* rows per phase (conv: M) */
-  /* stride-4 convT only, 0 otherwise: the rows are interleaved by phase (row m is phase m & 3 of
-     channel m >> 2; weights relaid by ptk_relayout_il / ptk_relayout16_il with il = C4), so the
-     four phases of an output column sit in one lane and go to four consecutive samples */
+  /* stride-4 convT only, 0 otherwise: the rows are interleaved by phase (a 32-row block holds the
+     four phases of eight channels; weights relaid by ptk_relayout_il with il = C4), so one
+     workgroup writes whole output lines and a lane four channels of one sample */
   int phase_il;
   int64_t q0, nq;             /* output columns [q0, q0 + nq) */
   /* Per-item column ranges (overlap-save windows compute only the columns their kept samples
@@ -131,6 +134,8 @@ typedef struct {
   float *y2;                  /* optional second output: LeakyReLU(a2) of every value stored in y,
                                  same index (the next conv's pre-activated input) */
   float a2;
+  void *ysp;                  /* optional output: the same LeakyReLU(a2) as split planes
+                                 [rows/8][2][ldy][8], batch stride bsy floats */
   int64_t ldy, bsy;
   int ys, ypad;
   int64_t Lout;
@@ -139,17 +144,15 @@ typedef struct {
   ptk_epi epi[PTK_MAX_EPI];
 } ptk_conv_desc;
 
-/* Relayout packed conv/convT weights [M/4][K][cin][4] into the MFMA operand layout
- * [Mp/32][K][cinp/8][64 lanes][4] (Mp = M rounded up to 32, zero rows/channels in the padding).  Returns the
- * cinp the kernels expect for this cin (ptk_conv_cinp). */
+/* Relayout packed conv/convT weights [M/4][K][cin][4] into what the conv kernel reads
+ * (ptk_kernels.hip, "weight relayout"): two fp16 parts of every weight, the fp32 weights, and a
+ * factor per row, ptk_relayout_floats floats in all, 16-byte aligned.  ptk_conv_cinp: the channel
+ * count the kernel expects for this cin. */
 int ptk_conv_cinp(int cin);
 size_t ptk_relayout_floats(int M, int K, int cin);
 int ptk_relayout(float *dst, const float *wp, int M, int K, int cin, void *s);
-/* the copy for 16-row tiles: [Mp/16][K][cinp/8][64][2], Mp = M rounded up to 16 */
-size_t ptk_relayout16_floats(int M, int K, int cin);
-int ptk_relayout16(float *dst, const float *wp, int M, int K, int cin, void *s);
-/* the same two layouts with a stride-4 convT's rows interleaved by phase (il = its rows per
-   phase C4, M = 4 * il): relaid row m is packed row (m & 3) * il + (m >> 2) */
+/* the same with a stride-4 convT's rows interleaved by phase: il = its rows per phase C4, a multiple
+   of 8, M = 4 * il */
 int ptk_relayout_il(float *dst, const float *wp, int M, int K, int cin, int il, void *s);
 int ptk_relayout16_il(float *dst, const float *wp, int M, int K, int cin, int il, void *s);
 /* fp16 -> fp32 expansion of n items (bit-exact: subnormals keep their value, inf / NaN keep sign
@@ -184,6 +187,9 @@ int ptk_leaky(const float *a, float *y, int64_t n, float alpha, void *s);
 /* y = leaky(((a + b) + c) / 3, alpha): the MRF branch average (ref/v21_graph_trace.txt:3851-3869) */
 int ptk_avg3_leaky(const float *a, const float *b, const float *c, float *y, int64_t n, float alpha,
                    void *s);
+/* the same over rows x T (rows a multiple of 8: items x channels), also written as split planes */
+int ptk_avg3_leaky_split(const float *a, const float *b, const float *c, float *y, void *ysp,
+                         int64_t rows, int64_t T, float alpha, void *s);
 
 /* decoder tail: conv_post output p [72][L] (row stride ldp) -> wav [16*(L-1)] (iSTFT + PQMF) */
 int ptk_tail(const float *p, int64_t ldp, int64_t L, float *wav, const float *consts, void *s);

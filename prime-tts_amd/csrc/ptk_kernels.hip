@@ -355,57 +355,149 @@ extern "C" int ptk_graph_destroy(void *exec) {
 }
 
 // ------------------------------------------------------------------------------ weight relayout
+// The conv kernel multiplies fp32 operands on the fp16 matrix cores: an operand v, scaled by a
+// power of two into fp16's range, is taken as two fp16 parts
+//     hi = fp16(v),  lo = fp16(v - hi),
+// each rounded to nearest even (v - hi is exact in fp32).  hi + lo differs from v by at most 2^-24
+// of it while lo stays a normal fp16, half a unit in fp32's last place, and by 2^-25 absolute below
+// that.  Weights are scaled row by row so that the row's largest magnitude lies in [2^14, 2^15):
+// the absolute part is then 2^-39 of the row's largest weight.  Inputs take the fixed scale
+// 2^CONV_XS (see conv_mfma_kernel for the columns whose inputs do not fit).
+//
 // Packed [M/4][K][cin][4] (the reference's conv layout; a convT's phase rows are just more rows)
-// -> MFMA operand layout [Mp/32][K][cinp/8][64][4].  For a row block mb, tap k and a chunk of 8
-// input channels, lane l = 32*h + r of a wave holds the four floats
-//     W[mb*32 + r][k][chunk*8 + 2*p + h],   p = 0..3,
-// which are exactly its A operands (row r, reduction index h) of the four v_mfma_f32_32x32x2_f32
-// that consume channel pairs (2p, 2p+1) of the chunk.  One 16-byte load per lane therefore feeds
-// four MFMAs, and the 1 KiB a wave loads for one (tap, chunk) is contiguous.  cinp rounds cin up
-// so every wave of the 4-way channel split owns whole chunks; padding rows/channels are zero.
-#define CONV_CK 8          // input channels per staged chunk (per wave)
-#define CONV_WAVES 4       // waves per workgroup, each owning a quarter of the channels
+// -> three parts, one after the other (Mp: M rounded up to 32, cinp: cin rounded up to 16; padding
+// rows and channels are zero):
+//   fp16 [Mp/32][cinp/16][K][2][64][8]: for a row block mb, a chunk of 16 input channels and a tap k,
+//     lane l = 32*h + r of a wave holds, of hi and of lo, the eight scaled values
+//     W[mb*32 + r][k][chunk*16 + 8*h + e], e = 0..7: its A operand of one v_mfma_f32_32x32x16_f16.
+//     One 16-byte load per lane and part; the 2 KiB a wave loads for one (chunk, tap) are
+//     contiguous and so are the taps of its chunks.
+//   fp32 [Mp/32][cinp/16][K][64][8]: the weights themselves in the same order (conv_mfma_kernel's
+//     second pass).
+//   fp32 [Mp]: per row, the factor 2^-(row exponent + CONV_XS) that takes a sum of products of scaled
+//     operands back; NaN for a row that has no fp16 form (an inf or NaN weight, or all of it below
+//     2^-100).
+#define CONV_CK 16         // input channels per staged chunk (per wave)
+#define CONV_TAPB 2048     // bytes of one (row block, chunk, tap) of either copy of the weights
+// Waves per SIMD the registers are budgeted for, and (chunk, tap) slices the A operands are loaded
+// ahead, by column blocks per wave.  A launch small enough for one column block (choose_tiles) has
+// about one wave per SIMD and waits for its loads, so it runs further ahead instead.
+#ifndef CONV_WPE1
+#define CONV_WPE1 3
+#define CONV_PD1 4
+#define CONV_WPE2 3
+#define CONV_PD2 4
+#endif
+#define CONV_XS 6          // the inputs' scale, 2^CONV_XS
 
-extern "C" int ptk_conv_cinp(int cin) {
-  const int q = CONV_WAVES * CONV_CK;
-  return (cin + q - 1) / q * q;
-}
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+extern "C" int ptk_conv_cinp(int cin) { return (cin + CONV_CK - 1) / CONV_CK * CONV_CK; }
 extern "C" size_t ptk_relayout_floats(int M, int K, int cin) {
   const size_t Mp = (size_t) (M + 31) / 32 * 32;
-  return Mp * (size_t) K * (size_t) ptk_conv_cinp(cin);
+  return Mp * (size_t) K * (size_t) ptk_conv_cinp(cin) * 2 + Mp;
 }
 
-// il: 0, or the rows per phase C4 of a stride-4 convT whose rows the MFMA layout interleaves by
-// phase: relaid row m is packed row (m & 3) * il + (m >> 2), phase m & 3 of channel m >> 2.
-__device__ __forceinline__ int relayout_row(int m, int il) { return il ? (m & 3) * il + (m >> 2) : m; }
+// two floats -> their fp16s (round to nearest even) in one word, a in the low half
+__device__ __forceinline__ unsigned f16_pair(float a, float b) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, h2{(_Float16) a, (_Float16) b});
+}
+// the two parts of a pair of floats
+__device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &l) {
+  const _Float16 ha = (_Float16) a, hb = (_Float16) b;
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  h = __builtin_bit_cast(unsigned, h2{ha, hb});
+  l = f16_pair(__builtin_fmaf((float) ha, -1.0f, a), __builtin_fmaf((float) hb, -1.0f, b));
+}
 
-__global__ void relayout_kernel(float *__restrict__ dst, const float *__restrict__ wp, int M,
-                                int K, int cin, int cinp, long long total, int il) {
-  long long i = (long long) blockIdx.x * blockDim.x + threadIdx.x;
-  const long long st = (long long) gridDim.x * blockDim.x;
-  const int nchunk = cinp / CONV_CK;
-  for (; i < total; i += st) {
-    const int p = (int) (i & 3);
-    const int lane = (int) ((i >> 2) & 63);
-    long long r = i >> 8;
-    const int chunk = (int) (r % nchunk);
-    r /= nchunk;
-    const int k = (int) (r % K);
-    const int mb = (int) (r / K);
-    const int m = mb * 32 + (lane & 31);
-    const int ci = chunk * CONV_CK + 2 * p + (lane >> 5);
-    float v = 0.0f;
-    if (m < M && ci < cin) {
-      const int ms = relayout_row(m, il);
-      v = wp[(((long long) (ms >> 2) * K + k) * cin + ci) * 4 + (ms & 3)];
+// Split planes: an activation tensor [C][T] already in two parts, scaled by 2^CONV_XS, as
+// [C/8][2][T][8] fp16: per group of eight channels the hi row and the lo row, a column's eight
+// channels in 16 bytes.  A conv reads it by copying 16-byte columns into its window, without the
+// conversions every row block would repeat.  Same bytes as the fp32 tensor.
+//
+// il: 0, or the rows per phase C4 (a multiple of 8) of a stride-4 convT whose rows the MFMA layout
+// interleaves by phase: a 32-row block holds eight channels, relaid row m is phase (m >> 3) & 3 of
+// channel (m >> 5) * 8 + (m & 7), packed row phase * il + channel.
+//
+// One workgroup per four packed rows, which are contiguous: their largest magnitudes first, then
+// (from cache) thread by thread eight channels of one (tap, chunk half) of the four rows.
+#define RELAY_THREADS 256
+__global__ void __launch_bounds__(RELAY_THREADS) relayout_kernel(
+    float *__restrict__ dst, const float *__restrict__ wp, int M, int K, int cin, int cinp, int il) {
+  __shared__ unsigned smax[4];
+  const int Mp = (M + 31) / 32 * 32, nchunk = cinp / CONV_CK;
+  const int tid = threadIdx.x, m0 = blockIdx.x * 4;
+  const float4 *src = reinterpret_cast<const float4 *>(wp) + (long long) blockIdx.x * K * cin;
+  if (tid < 4) smax[tid] = 0;
+  __syncthreads();
+  if (m0 < M) {
+    unsigned mx[4] = {0, 0, 0, 0};   // as bit patterns: inf and NaN sort above every finite value
+    for (int i = tid; i < K * cin; i += RELAY_THREADS) {
+      const float4 v = src[i];
+      mx[0] = max(mx[0], __float_as_uint(v.x) & 0x7fffffffu);
+      mx[1] = max(mx[1], __float_as_uint(v.y) & 0x7fffffffu);
+      mx[2] = max(mx[2], __float_as_uint(v.z) & 0x7fffffffu);
+      mx[3] = max(mx[3], __float_as_uint(v.w) & 0x7fffffffu);
     }
-    dst[i] = v;
+#pragma unroll
+    for (int r = 0; r < 4; r++) atomicMax(&smax[r], mx[r]);
+  }
+  __syncthreads();
+  float up[4];
+  int row[4];   // relaid rows
+  const long long wn = (long long) Mp * K * cinp;
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int ms = m0 + r;
+    const int c = il ? ms % il : 0;
+    row[r] = il && ms < M ? (c >> 3) * 32 + ms / il * 8 + (c & 7) : ms;
+    const unsigned mx = smax[r];
+    const int e = (int) (mx >> 23) - 127;   // exponent of the largest magnitude
+    const bool none = mx == 0, bad = !none && (e < -100 || mx >= 0x7f800000u);
+    const int s = none || bad ? 0 : 14 - e;
+    up[r] = __uint_as_float((unsigned) (127 + s) << 23);
+    if (tid == 0)
+      dst[2 * wn + row[r]] = bad ? __uint_as_float(0x7fc00000u) : __uint_as_float((unsigned) (127 - s - CONV_XS) << 23);
+  }
+  for (int i = tid; i < nchunk * K * 2; i += RELAY_THREADS) {
+    const int h = i & 1, k = (i >> 1) % K, chunk = (i >> 1) / K;
+    float v[4][8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const int ci = chunk * CONV_CK + 8 * h + e;
+      const float4 f = m0 < M && ci < cin ? src[(long long) k * cin + ci] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      v[0][e] = f.x;
+      v[1][e] = f.y;
+      v[2][e] = f.z;
+      v[3][e] = f.w;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const long long slice = ((long long) (row[r] >> 5) * nchunk + chunk) * K + k;
+      const int lane = 32 * h + (row[r] & 31);
+      u32x4 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        unsigned a, b;
+        split_pair(v[r][2 * e] * up[r], v[r][2 * e + 1] * up[r], a, b);
+        hi[e] = a;
+        lo[e] = b;
+      }
+      u32x4 *d16 = reinterpret_cast<u32x4 *>(dst) + slice * (CONV_TAPB / 16) + lane;
+      d16[0] = hi;
+      d16[64] = lo;
+      float4 *d32 = reinterpret_cast<float4 *>(dst + wn) + slice * (CONV_TAPB / 16) + lane * 2;
+      d32[0] = make_float4(v[r][0], v[r][1], v[r][2], v[r][3]);
+      d32[1] = make_float4(v[r][4], v[r][5], v[r][6], v[r][7]);
+    }
   }
 }
 
 static int relayout_il_ok(int M, int il, const char *who) {
-  if (il != 0 && (il < 1 || M != 4 * il)) {
-    set_err("%s: phase interleave needs M = 4 x rows per phase (M %d, rows per phase %d)", who, M, il);
+  if (il != 0 && (il < 1 || M != 4 * il || il % 8 != 0)) {
+    set_err("%s: phase interleave needs M = 4 x rows per phase, a multiple of 8 (M %d, rows per phase %d)", who, M, il);
     return 0;
   }
   return 1;
@@ -413,64 +505,17 @@ static int relayout_il_ok(int M, int il, const char *who) {
 
 extern "C" int ptk_relayout_il(float *dst, const float *wp, int M, int K, int cin, int il, void *s) {
   if (!relayout_il_ok(M, il, "ptk_relayout_il")) return -1;
-  const long long total = (long long) ptk_relayout_floats(M, K, cin);
-  long long blocks = (total + 255) / 256;
-  if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(relayout_kernel, dim3((unsigned) blocks), dim3(256), 0, (hipStream_t) s, dst,
-                     wp, M, K, cin, ptk_conv_cinp(cin), total, il);
+  hipLaunchKernelGGL(relayout_kernel, dim3((unsigned) ((M + 31) / 32 * 8)), dim3(RELAY_THREADS), 0,
+                     (hipStream_t) s, dst, wp, M, K, cin, ptk_conv_cinp(cin), il);
   HCHK(hipGetLastError());
   return 0;
 }
 extern "C" int ptk_relayout(float *dst, const float *wp, int M, int K, int cin, void *s) {
   return ptk_relayout_il(dst, wp, M, K, cin, 0, s);
 }
-
-// The same weights for 16-row tiles on v_mfma_f32_16x16x4_f32: [Mp/16][K][cinp/8][64][2] (Mp = M
-// rounded up to 16).  Lane l = 16*kq + r holds W[mb*16 + r][k][chunk*8 + 4*s + kq], s = 0, 1: its
-// A operands (row r, reduction index kq) of the two MFMAs that consume channels 4s .. 4s + 3 of
-// the chunk.  One 8-byte load per lane feeds both, and a wave's (tap, chunk) slice is 512
-// contiguous bytes.
-extern "C" size_t ptk_relayout16_floats(int M, int K, int cin) {
-  const size_t Mp = (size_t) (M + 15) / 16 * 16;
-  return Mp * (size_t) K * (size_t) ptk_conv_cinp(cin);
-}
-
-__global__ void relayout16_kernel(float *__restrict__ dst, const float *__restrict__ wp, int M,
-                                  int K, int cin, int cinp, long long total, int il) {
-  long long i = (long long) blockIdx.x * blockDim.x + threadIdx.x;
-  const long long st = (long long) gridDim.x * blockDim.x;
-  const int nchunk = cinp / CONV_CK;
-  for (; i < total; i += st) {
-    const int s = (int) (i & 1);
-    const int lane = (int) ((i >> 1) & 63);
-    long long r = i >> 7;
-    const int chunk = (int) (r % nchunk);
-    r /= nchunk;
-    const int k = (int) (r % K);
-    const int mb = (int) (r / K);
-    const int m = mb * 16 + (lane & 15);
-    const int ci = chunk * CONV_CK + 4 * s + (lane >> 4);
-    float v = 0.0f;
-    if (m < M && ci < cin) {
-      const int ms = relayout_row(m, il);
-      v = wp[(((long long) (ms >> 2) * K + k) * cin + ci) * 4 + (ms & 3)];
-    }
-    dst[i] = v;
-  }
-}
-
+// (one layout serves every tile; the name stays for callers that have it)
 extern "C" int ptk_relayout16_il(float *dst, const float *wp, int M, int K, int cin, int il, void *s) {
-  if (!relayout_il_ok(M, il, "ptk_relayout16_il")) return -1;
-  const long long total = (long long) ptk_relayout16_floats(M, K, cin);
-  long long blocks = (total + 255) / 256;
-  if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(relayout16_kernel, dim3((unsigned) blocks), dim3(256), 0, (hipStream_t) s,
-                     dst, wp, M, K, cin, ptk_conv_cinp(cin), total, il);
-  HCHK(hipGetLastError());
-  return 0;
-}
-extern "C" int ptk_relayout16(float *dst, const float *wp, int M, int K, int cin, void *s) {
-  return ptk_relayout16_il(dst, wp, M, K, cin, 0, s);
+  return ptk_relayout_il(dst, wp, M, K, cin, il, s);
 }
 
 // ------------------------------------------------------------------------------ fp16 expansion
@@ -545,42 +590,59 @@ __device__ __forceinline__ int fdiv(int n, FastDiv f) {
   return (int) (((unsigned long long) (unsigned) n * f.m) >> f.s);
 }
 
-// Per-problem launch facts computed on the host, 64 bytes: one scalar load at kernel entry.
+// Per-problem launch facts computed on the host: what a workgroup needs up to its first loads, in
+// 32 bits and in one batch of scalar loads at kernel entry.
 struct ConvProb {
   int count;                      // workgroups of the problem (grid row blockIdx.y = problem)
-  int mt;                         // RB-row blocks
-  int nt;                         // column tiles of a middle batch item
-  int nt0;                        // of item 0 (its columns start ext_l earlier; one item: all)
-  int ntl;                        // of the last item (its columns end ext_r later)
-  int nitem;                      // batch items
-  FastDiv div_tiles;              // by mt * nt (tiles of a middle batch item)
+  int mt;                         // 32-row blocks
+  int mtnt, mtnt0;                // mt x column tiles of a middle batch item / of item 0 (its columns
+                                  // start ext_l earlier; one item: all of them)
+  int last;                       // batch items - 1
+  FastDiv div_tiles;              // by mtnt
   FastDiv div_mt;                 // by mt
-  FastDiv div_phase;              // by C4 / RB (row blocks per convT phase) when one_phase
-  int flags;                      // PROB_ONE_PHASE | PROB_FAST | PROB_PHASE_IL
+  FastDiv div_phase;              // by C4 / 32 (row blocks per convT phase) when one_phase, else 0
+  int flags;                      // PROB_*
   int ext_l;                      // item 0's first column is q0 - ext_l
   int addt;                       // the chain's first tensor add, or -1
   int M;                          // GEMM rows
+  int q0;
+  const void *x;                  // what the windows are loaded from (ptk_conv_desc x or xsp)
+  const void *w;                  // fp16 weights
+  const float *scale;             // their row factors
+  const float *bias;
+  int nbias4;                     // bytes of the bias
+  int C4;
+  int K, dil, st, cin, nchunk, ldx4, lim, shift;   // ldx4: input row stride in bytes
+  long long bsx;
+  int kd, xw;                     // (K - 1) * dil; window columns
+  float in_a;
+  int wslots;                     // ConvGroup's: LDS of one wave, in 16-byte slots
+  int pad[8];
 };
-// every row block lies inside one phase (conv, or C4 % RB == 0)
+// every row block lies inside one phase (conv, or C4 % 32 == 0)
 #define PROB_ONE_PHASE 1
 // output / residual index ranges fit the 32-bit epilogue
 #define PROB_FAST 2
-// stride-4 convT with its rows interleaved by phase (row m: phase m & 3 of channel m >> 2)
+// stride-4 convT with its rows interleaved by phase (row m: phase (m >> 3) & 3 of channel
+// (m >> 5) * 8 + (m & 7))
 #define PROB_PHASE_IL 4
-static_assert(sizeof(ConvProb) == 64, "one 64-byte scalar load");
+// virtual input column 0 reads column 1, column c > 0 reads column c - 1
+#define PROB_REFLECT 8
+static_assert(sizeof(ConvProb) == 192, "three 64-byte scalar loads");
 
 // What the fast epilogue reads, 128 bytes per problem, fetched in one batch of scalar loads when
 // the epilogue starts (field by field from the descriptor, each chain op's fields had been a
 // scalar load and a wait of their own).
 struct ConvEpi {
   const float *y, *y2, *t;        // output, its LeakyReLU copy (or null), the residual of op addt
+  const void *ysp;                // its LeakyReLU copy as split planes (or null)
   long long bsy, bst;             // batch strides of y / y2 and of t
   int ldy, ldt;                   // row strides (fit 32 bits on the fast path)
   int lout, qend, ext_r, ys, ypad, C4, nepi;   // qend: a middle item's column end
   int ops;                        // op e in bits 4e .. 4e + 3
   float a[PTK_MAX_EPI];
   float a2;
-  int pad[7];
+  int pad[5];
 };
 static_assert(sizeof(ConvEpi) == 128, "two 64-byte scalar loads");
 
@@ -589,37 +651,21 @@ struct ConvGroup {
   ConvEpi ep[PTK_MAX_GROUP];
   ptk_conv_desc d[PTK_MAX_GROUP];
   int ngroup;
-  int split;                      // waves of a workgroup sharing one output block: 1, 2, 4 or 8
-  int lg_split;                   // log2(split)
+  int wslots;                     // LDS of one wave, in 16-byte slots
+  int wcols;                      // window columns staged (32 * units)
 };
 
-// Staged input window of one chunk (8 channels): NB column blocks of 32 outputs need
-// (32*NB - 1)*stride + |K-1|*|dil| + 1 columns; the kernel supports up to 64*(NB+1).  LDS holds it
-// as two planes h = 0, 1 of float4 columns: plane h, column c = channels h, 2+h, 4+h, 6+h.  The
-// four B operands a lane (column, h) needs for one tap are then one 16-byte LDS read, and each
-// half-wave reads (and each staging store writes) consecutive 16-byte columns: no bank conflicts.
-template <int NB> struct WinGeo {
-  static constexpr int NJ = NB + 1;          // 64-column slices a lane loads per row
-  static constexpr int XWMAX = 64 * NJ;
-};
-
-// 16-row tiles (RB = 16) keep the same window but store it as four planes q = 0..3 of float2
-// columns: plane q, column c = channels q, 4 + q, the B operands (reduction index q) of the two
-// 16x16x4 MFMAs of a chunk.  A quarter-wave reads 16 consecutive float2 of one plane per tap and
-// column block; planes are XWMAX + 16 float2 apart, so the two quarter-waves served together
-// fall on different banks.
-//
-// LDS of one workgroup: per wave its staging area, and the partial-sum area (the staging area
-// itself when the partial sums fit in it).
-template <int NB, int RB, int NW> struct LdsGeo {
-  static constexpr int XWMAX = WinGeo<NB>::XWMAX;
-  static constexpr int PS = RB == 32 ? XWMAX : XWMAX + 16;   // plane stride (float4 / float2)
-  static constexpr int STG = 8 * PS;                         // staging floats per wave
-  static constexpr int NV = RB / 2;                          // accumulators per lane and column block
-  static constexpr int RED = NB * NV * 64;                   // partial-sum floats per wave
-  static constexpr bool OWN_RED = RED <= STG;
-  static constexpr size_t BYTES = (size_t) NW * (STG > RED ? STG : RED) * sizeof(float);
-};
+// Staged input window of one chunk (16 channels): NB column blocks of 32 outputs need
+// (32*NB - 1)*stride + |K-1|*|dil| + 1 columns, staged as NU units of 32 columns (NU <= 4).  LDS
+// holds it as planes [part][h] of 16-byte columns: plane (part, h), column c = that part of
+// channels 8h .. 8h + 7.  The B operand a lane (column, h) needs for one tap and part is then one
+// 16-byte LDS read, and each half-wave reads (and each staging store writes) consecutive 16-byte
+// columns: no bank conflicts.
+#define CONV_NU_MAX 4
+// 16-byte LDS slots of one wave: its window / its partial sums
+static constexpr int conv_slots(int nu, int nb) { return nu * 32 * 4 > nb * 256 ? nu * 32 * 4 : nb * 256; }
+// and of the workgroup: one flag per wave, one magnitude per window column
+#define CONV_EXTRA_SLOTS (2 + CONV_NU_MAX * 8)
 
 // word 3 of a raw buffer resource on gfx9-family parts (gfx950): 32-bit data, range checked
 #define PTK_BUF_WORD3 0x00020000
@@ -639,371 +685,488 @@ __device__ __forceinline__ float buf_load(__amdgpu_buffer_rsrc_t r, unsigned vof
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
 
-// One workgroup = NW waves (4, or 8 for the 8-way split).  The waves form NW/S column groups of S
-// waves; the S waves of a group compute the same RB-row x 32*NB-column output block over disjoint
-// eighths/quarters/halves of the input channels (S = 1: each wave its own block over all channels)
-// and are reduced through LDS in wave order (deterministic).  NW = 8 runs S = 8 only.  KT > 0:
-// every problem of the group has K <= KT and the whole next chunk's A operands (KT float4 / float2
-// per lane) are prefetched while the current chunk runs; KT == 0: any K, A loaded per tap.  IN:
-// input transform (PTK_IN_*).  RB: rows per tile, 32 (32x32x2 MFMA, weights from d.w) or 16
-// (16x16x4 MFMA on two 16-column blocks, weights from d.w16).
-template <int KT, int NB, int IN, int RB, int NW>
-__global__ void __launch_bounds__(64 * NW) conv_mfma_kernel(const ConvGroup g) {
-  extern __shared__ float smem[];
-  static_assert(RB == 32 || (RB == 16 && NB == 1), "16-row tiles are built for one column block");
-  static_assert(NW == 4 || (NW == 8 && NB == 1), "8-wave workgroups are built for one column block");
-  constexpr int NJ = WinGeo<NB>::NJ, XWMAX = WinGeo<NB>::XWMAX;
-  using Geo = LdsGeo<NB, RB, NW>;
-  constexpr int PS = Geo::PS, NV = Geo::NV;
+// the two parts of one lane's A or B operand
+struct Parts {
+  f16x8 h, l;
+};
+
+// max(m, |a|, |b|); NaN if any of them is
+__device__ __forceinline__ float max_mag(float m, float a, float b) {
+  asm("v_maximum3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));
+  return m;
+}
+__device__ __forceinline__ float half_of(unsigned pair, int i) {
+  return (float) __builtin_bit_cast(_Float16, (unsigned short) (pair >> (16 * i)));
+}
+// The largest input magnitude m of a receptive field for which the scaled fp16 parts hold the inputs
+// to 2^-24 of m: neither too large for fp16 nor so small that lo loses bits (all zero is exact).
+__device__ __forceinline__ bool conv_fits(float m) {
+  const float h = (float) (_Float16) (m * (float) (1 << CONV_XS));
+  return m == 0.0f || (h >= 0.25f && h <= 65504.0f);
+}
+// what the first pass tests on the fly: false wherever conv_fits is
+__device__ __forceinline__ bool conv_alarm_free(float m) {
+  return m < 1023.0f && (m >= 0.00390625f || m == 0.0f);
+}
+
+// One workgroup = S waves on one block of 32 rows x 32*NB columns.  The waves take disjoint runs of
+// the 16-channel chunks and are reduced through LDS in wave order (deterministic).  Each product of
+// two fp32 values is taken as three fp16 products on v_mfma_f32_32x32x16_f16 (hi.lo, lo.hi, hi.hi;
+// lo.lo is below 2^-24 of it), accumulated in fp32.
+//
+// An output column whose inputs (the receptive field, all channels) conv_fits refuses, and every
+// column of a row block with a weight that has no fp16 form, is computed by a second pass over the
+// block on v_mfma_f32_32x32x2_f32 instead, from the fp32 operands.  Which pass an output comes from
+// depends on its own receptive field only, not on the tile or batch it is computed in.  The first
+// pass watches the magnitudes it stages (a unit's own channels, so it may raise a false alarm but
+// misses nothing); only a workgroup it alarms looks at its columns one by one.
+//
+// KT: the taps the straight-line bodies are built for (11: K = 11, 7 and 3; 4: K = 4, the convT
+// phase form); any other K goes through a rolled loop.  IN: input transform (PTK_IN_*).
+template <int KT, int NB, int IN, int S>
+__global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(NB == 1 ? CONV_WPE1 : CONV_WPE2)))
+conv_mfma_kernel(const ConvGroup g) {
+  extern __shared__ u32x4 smem[];
   // Grid row blockIdx.y is the problem, so every field of it can be fetched at entry; rows are
   // as long as the largest problem's workgroup count, and the excess of a shorter one exits.
   const int p = blockIdx.y;
   const ConvProb pi = g.info[p];
-  const ptk_conv_desc &d = g.d[p];
-  // The scalar-cache lines of the problem's descriptor fields the prologue reads (x .. q0) and of
-  // the split are touched in the same batch of loads as the launch facts: the prologue's later
-  // reads of them then hit, instead of each batch waiting out a round trip of its own.
-  asm volatile("" ::"s"(pi.count), "s"(d.x), "s"(d.w16), "s"(d.q0), "s"(g.split));
-  const int bid = blockIdx.x;
+  // (a field of each scalar-cache line, so that all loads go out together, ahead of the test)
+  asm volatile("" ::"s"(pi.count), "s"(pi.x), "s"(pi.shift), "s"(pi.wslots));
+  const int bid = blockIdx.x, wslots = pi.wslots;
   if (bid >= pi.count) return;
-  const int mt = pi.mt;
-  // Tiles item after item, column tile after column tile, row block fastest: item 0 has nt0
-  // column tiles, the middle items nt, the last one ntl >= nt (all nt for a plain launch).
-  // Written as masks and min / max rather than selects, which the compiler turns into branches
-  // around the divisions (measured slower on single-wave-per-SIMD launches).
-  const int c0 = mt * pi.nt0, t = bid - c0;
+  // Tiles item after item, column tile after column tile, row block fastest: item 0 has its own
+  // number of column tiles, the last one takes the extra ones.  Written as masks and min / max
+  // rather than selects, which the compiler turns into branches around the divisions (measured
+  // slower on single-wave-per-SIMD launches).
+  const int t = bid - pi.mtnt0;
   const int past0 = ~(t >> 31);                          // -1 past item 0's tiles, else 0
   const int bq = fdiv(max(t, 0), pi.div_tiles);
-  const int b = min(bq + 1, pi.nitem - 1) & past0;      // the last item takes its extra tiles
-  const int r = bid - ((c0 + (b - 1) * (mt * pi.nt)) & past0);
+  const int b = min(bq + 1, pi.last) & past0;            // the last item takes its extra tiles
+  const int r = bid - ((pi.mtnt0 + (b - 1) * pi.mtnt) & past0);
   const int tn = fdiv(r, pi.div_mt);
-  const int mb = r - tn * mt;
-  const bool last_item = b == pi.nitem - 1;
-  const long long q0i = d.q0 - (long long) (pi.ext_l & ~past0);   // this item's first column
-  const int S = g.split, lgS = g.lg_split, G = NW >> lgS;
+  const int mb = r - tn * pi.mt;
+  const bool last_item = b == pi.last;
+  const int q0 = pi.q0 - (pi.ext_l & ~past0) + tn * (32 * NB);   // this block's first column
 
-  // descriptor fields used in loops, read once (the problem index is dynamic, so the compiler
-  // would otherwise re-read them from the kernel arguments)
-  const int K = d.K, dil = d.dil, st = d.stride, cin = d.cin;
-  const unsigned ldx4 = (unsigned) d.ldx * 4u;
-  const long long lim = d.lim;
-  const float in_a = d.in_a;
-  const int nchunk = d.cinp / CONV_CK;          // chunks over all channels
-  const int nch = nchunk >> lgS;                // chunks of this wave
+  const int K = pi.K, dil = pi.dil, st = pi.st, cin = pi.cin, nchunk = pi.nchunk, lim = pi.lim;
+  const unsigned ldx4 = (unsigned) pi.ldx4;
+  const float in_a = pi.in_a;
 
   const int lane = threadIdx.x & 63;
   // wave index: uniform across the wave, which the compiler cannot see on its own (without this
   // the wave-based buffer resources would be treated as divergent)
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ks = w & (S - 1), cg = w >> lgS;    // channel split index, column group
+  const int chunk0 = w * nchunk / S, nch = (w + 1) * nchunk / S - chunk0;   // chunks of this wave
   // The phase of this row block (convT: row m is phase m / C4 of channel m % C4), when the block
   // lies inside one phase.
-  const bool phase_rows = d.C4 != d.M;
   const bool one_phase = (pi.flags & PROB_ONE_PHASE) != 0;
-  // rows interleaved by phase: only the 4-tap convT phase form (KT = 4) carries that code, so the
-  // other instantiations compile exactly as without it (the launcher refuses it elsewhere)
+  // rows interleaved by phase: only the 4-tap convT phase form (KT = 4) carries that code (the
+  // launcher refuses it elsewhere)
   const bool phase_il = KT == 4 && (pi.flags & PROB_PHASE_IL) != 0;
-  const int r_tile = phase_rows && one_phase ? fdiv(mb, pi.div_phase) : 0;
-  // Lane l < RB loads the bias of the block's row l once the first chunk's loads are in flight,
-  // and the epilogue fetches each value's bias from the lane of its row (ds_bpermute): the load's
-  // latency is spent behind the main loop, and no wave depends on another's write.
-  float bias_r = 0.0f;
+  const int r_tile = fdiv(mb, pi.div_phase);
+  // Every lane loads the bias and the scale of row lane & 31 of the block, once the first chunk's
+  // loads are in flight, and the epilogue fetches each value's from the lane of its row
+  // (ds_bpermute): the loads' latency is spent behind the main loop, and no wave depends on
+  // another's write.  A row without a bias is past the buffer and reads 0.
+  float bias_r = 0.0f, scale_r = 1.0f;
   auto load_bias = [&]() {
-    // the fields read in one batch ahead of any branch (under the kernel's scalar-register
-    // pressure the compiler re-reads kernel arguments where they are used, one wait per read)
-    const float *bp = d.bias;
-    const int nbias = d.nbias, Mr = d.M, C4r = d.C4;
-    const int m = mb * RB + lane;
-    int co = m - r_tile * C4r;   // conv: r_tile = 0
-    if (phase_il) co = m >> 2;
-    else if (!one_phase) co = m % C4r;
-    if (lane < RB && bp != nullptr && m < Mr && co < nbias) bias_r = bp[co];
+    const int l = lane & 31;
+    int co = mb * 32 - r_tile * pi.C4 + l;   // conv: r_tile = 0
+    if (phase_il) co = mb * 8 + (l & 7);
+    else if (!one_phase) co = (mb * 32 + l) % pi.C4;
+    bias_r = buf_load(__builtin_amdgcn_make_buffer_rsrc((void *) pi.bias, (short) 0, pi.nbias4, PTK_BUF_WORD3),
+                      (unsigned) co * 4u, 0);
+    scale_r = pi.scale[mb * 32 + l];
   };
-  // bias of row `row` of the block (every lane of the wave must be active)
+  // bias and scale of row `row` of the block (every lane of the wave must be active)
   auto bias_of = [&](int row) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(row * 4, __float_as_int(bias_r)));
   };
-  const int half = lane >> 5;     // RB = 32: which of the two reduction rows this lane feeds
+  auto scale_of = [&](int row) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(row * 4, __float_as_int(scale_r)));
+  };
+  const int half = lane >> 5;     // which eight of a chunk's channels this lane feeds
   const int l32 = lane & 31;
-  const int quad = lane >> 4;     // RB = 16: the reduction index (and row group) of this lane
-  const int l16 = lane & 15;
-  const int q0off = (tn * G + cg) * (32 * NB);   // this wave's first column past the item's first
-  const long long q0 = q0i + q0off;
-  const int kd = (K - 1) * dil;
-  const int dmin = kd < 0 ? kd : 0;
-  const int XW = (32 * NB - 1) * st + (kd < 0 ? -kd : kd) + 1;
-  const long long cmin = q0 * st + dmin - d.shift;
-  const int chunk0 = ks * nch;
-  float *xsw = smem + w * Geo::STG;   // this wave's staging planes
-  float4 *xs = reinterpret_cast<float4 *>(xsw);    // RB = 32: [h][column] float4
-  float2 *xs2 = reinterpret_cast<float2 *>(xsw);   // RB = 16: [q][column] float2
+  const int dmin = min(pi.kd, 0);
+  const int XW = pi.xw;
+  const int cmin = q0 * st + dmin - pi.shift;   // the window's first virtual column
+  u32x4 *const xs = smem + w * wslots;   // this wave's staging planes
 
-  // Window columns this lane stages, fixed for the wave: byte offset in the row, or an offset the
-  // buffer range check turns into 0 (columns outside [0, lim), past the window).  The row offset
-  // is wave-uniform and goes into the scalar offset.  A row past cin (zero padding of the last
-  // chunk when cin is not a multiple of 8) reads row 0 and is zeroed when it is stored.
-  const long long xoff = (long long) b * d.bsx;
+  // Window columns this lane stages, fixed for the wave: unit u, column 32u + l32, channels 8*half
+  // .. 8*half + 7 of the chunk; byte offset of the first, or an offset the buffer range check turns
+  // into 0 (columns outside [0, lim), past the window).  The row step and the chunk are wave-uniform
+  // and go into the scalar offset.
+  const long long xoff = b * pi.bsx;
   const unsigned nrec = (unsigned) cin * ldx4;
-  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-      (void *) (d.x + xoff), (short) 0, (int) nrec, PTK_BUF_WORD3);
-  unsigned voff[NJ];
+  unsigned voff[CONV_NU_MAX];
+  {
+    constexpr unsigned CB = IN == PTK_IN_SPLIT ? 16 : 4;   // bytes of a column of a row (or row group)
+    const unsigned h8 = half ? 8u * ldx4 : 0u;
+    int c = cmin + l32;
+    if (pi.flags & PROB_REFLECT) {   // (column 0 reads column 1: the window holds 0 and 1 together)
 #pragma unroll
-  for (int jj = 0; jj < NJ; jj++) {
-    const int col = lane + 64 * jj;
-    const long long c = cmin + col;
-    const bool ok = (col < XW) & (c >= 0) & (c < lim);
-    const long long pc = d.reflect_l1 ? (c == 0 ? 1 : c - 1) : c;
-    voff[jj] = ok ? (unsigned) pc * 4u : PTK_OOB;
+      for (int u = 0; u < CONV_NU_MAX; u++, c += 32)
+        voff[u] = (unsigned) c < (unsigned) lim && l32 + 32 * u < XW ? (unsigned) (c == 0 ? 1 : c - 1) * CB + h8 : PTK_OOB;
+    } else {
+#pragma unroll
+      for (int u = 0; u < CONV_NU_MAX; u++, c += 32)
+        voff[u] = (unsigned) c < (unsigned) lim && l32 + 32 * u < XW ? (unsigned) c * CB + h8 : PTK_OOB;
+    }
   }
 
-  // Staging is split so that all global loads of a chunk are in flight together: the load phase
-  // only issues loads, the store phase (one chunk later) transforms and writes LDS.
-  // Rows past cin exist only when cin is not a multiple of 32 (cinp > cin); MASK (compile time)
-  // selects the chunk code that handles them, so the common case carries no per-row tests.
-  // NJU (compile time) of the NJ slices are staged: windows up to 64 columns (every decoder conv
-  // but K = 11 at dilation 5) need one, which halves the window loads and LDS stores.
-  float pf[CONV_CK][NJ];
-  auto load_chunk = [&](int c0, auto mask, auto nju) {
-    constexpr bool MASK = decltype(mask)::value;
-    constexpr int NJU = decltype(nju)::value;
-#pragma unroll
-    for (int r = 0; r < CONV_CK; r++) {
-      const unsigned rowo = (!MASK || c0 + r < cin) ? (unsigned) (c0 + r) * ldx4 : 0u;
-#pragma unroll
-      for (int jj = 0; jj < NJU; jj++) {
-        pf[r][jj] = buf_load(rx, voff[jj], rowo);
-      }
-    }
-  };
-  auto store_chunk = [&](int c0, auto mask, auto nju) {
-    constexpr bool MASK = decltype(mask)::value;
-    constexpr int NJU = decltype(nju)::value;
-    const int nlive = cin - c0;   // rows of this chunk that hold channels
-#pragma unroll
-    for (int jj = 0; jj < NJU; jj++) {
-      float v[CONV_CK];
-#pragma unroll
-      for (int r = 0; r < CONV_CK; r++) {
-        v[r] = in_xform<IN>(pf[r][jj], in_a);
-      }
-      if constexpr (MASK) {
-        if (nlive < CONV_CK) {
-#pragma unroll
-          for (int r = 0; r < CONV_CK; r++) v[r] = r < nlive ? v[r] : 0.0f;
-        }
-      }
-      if constexpr (RB == 32) {
-        xs[lane + 64 * jj] = make_float4(v[0], v[2], v[4], v[6]);
-        xs[XWMAX + lane + 64 * jj] = make_float4(v[1], v[3], v[5], v[7]);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; q++) xs2[q * PS + lane + 64 * jj] = make_float2(v[q], v[4 + q]);
-      }
-    }
-  };
-
-  // accumulators: RB = 32, one 32x32 block per column block (16 values per lane); RB = 16, two
-  // 16x16 blocks per column block (4 values per lane each)
-  using AccT = std::conditional_t<RB == 32, f32x16, f32x4>;
-  constexpr int NCB = RB == 32 ? 1 : 2;
-  AccT acc[NB][NCB];
+  // accumulators: one 32x32 block per column block (16 values per lane)
+  f32x16 acc[NB];
 #pragma unroll
   for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-    for (int cb = 0; cb < NCB; cb++)
-#pragma unroll
-      for (int v = 0; v < NV / NCB; v++) acc[nb][cb][v] = 0.0f;
+    for (int v = 0; v < 16; v++) acc[nb][v] = 0.0f;
 
-  // A operands: float4 (RB = 16: float2) ((mb*K + k)*nchunk + chunk)*64 + lane of the relaid
-  // weights, read through a buffer resource based at this wave's first chunk: the lane offset is
-  // fixed and the (tap, chunk) offset is wave-uniform, so a load costs no vector address arithmetic
-  using AT = std::conditional_t<RB == 32, float4, float2>;
-  constexpr int ABYTES = 64 * (int) sizeof(AT);   // one (tap, chunk) slice of a wave
-  const AT *wbase = reinterpret_cast<const AT *>(RB == 32 ? d.w : d.w16) +
-                    ((long long) mb * K * nchunk + chunk0) * 64;
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
-      (void *) wbase, (short) 0, (int) ((unsigned) K * (unsigned) nchunk * (unsigned) ABYTES),
-      PTK_BUF_WORD3);
-  const unsigned wlane = (unsigned) lane * (unsigned) sizeof(AT);
-  const int wtap = nchunk * ABYTES;  // bytes between taps
-  auto wa = [&](int k, int j) {
-    if constexpr (RB == 32)
-      return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rw, wlane, k * wtap + j * ABYTES, 0));
-    else
-      return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rw, wlane, k * wtap + j * ABYTES, 0));
+  // A operands: the wave's (chunk, tap) slices are contiguous, read through a buffer resource based
+  // at its first chunk: the lane offset is fixed and the slice offset is wave-uniform, so a load
+  // costs no vector address arithmetic
+  const char *wbase = reinterpret_cast<const char *>(pi.w) +
+                      (long long) (mb * nchunk + chunk0) * (K * CONV_TAPB);
+  // (a resource with no records reads 0 and fetches nothing: the loads past the wave's last chunk)
+  auto w_rsrc = [&](bool live) {
+    return __builtin_amdgcn_make_buffer_rsrc(
+        (void *) wbase, (short) 0, live ? (int) ((unsigned) K * (unsigned) nch * (unsigned) CONV_TAPB) : 0,
+        PTK_BUF_WORD3);
   };
-  // staging-plane index of tap 0, column block 0 (float4 for RB = 32, float2 for RB = 16)
-  const int lbase = RB == 32 ? half * XWMAX + l32 * st - dmin : quad * PS + l16 * st - dmin;
+  auto x_rsrc = [&](bool live) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *) (reinterpret_cast<const float *>(pi.x) + xoff),
+                                             (short) 0, live ? (int) nrec : 0, PTK_BUF_WORD3);
+  };
+  const unsigned wlane = (unsigned) lane * 16u;
+  auto wa = [&](__amdgpu_buffer_rsrc_t rw, int slice) {
+    const int so = slice * CONV_TAPB;
+    Parts a;
+    a.h = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rw, wlane, so, 0));
+    a.l = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rw, wlane + 1024u, so, 0));
+    return a;
+  };
 
-  // the MFMAs of one tap: xr points at this lane's B operands of column block 0 (a float4 of
-  // plane h for RB = 32, a float2 of plane quad for RB = 16)
-  auto mfma4 = [&](const AT a, const auto *xr) {
-    if constexpr (RB == 32) {
+  // The chunk loop, for a compile-time tap count KC (0: runtime K) and NU window units.  A chunk's
+  // window goes through three stages: its loads are issued while the chunk two before it runs, its
+  // split (32 VALU instructions a unit) runs between the MFMAs of the chunk before it, which hide up
+  // to six VALU instructions each (measured: 12 MFMAs 181 ns, with 72 VALU between them 185 ns), and
+  // only the LDS stores stand between two chunks.  Rows past cin exist only when cin is not a
+  // multiple of 16; MASK (compile time) selects the code that handles them.
+  bool odd = false;   // a magnitude conv_fits refuses was staged by this lane
+  auto run = [&](auto kc, auto mask, auto nuc) {
+    constexpr int KC = decltype(kc)::value, NU = decltype(nuc)::value;
+    constexpr bool MASK = decltype(mask)::value;
+    constexpr int PS = NU * 32;   // plane stride (16-byte slots)
+    constexpr int PD = KC == 0 ? 1 : NB == 1 ? CONV_PD1 : CONV_PD2;   // slices the A operands are loaded ahead of their use
+    constexpr bool SPLIT = IN == PTK_IN_SPLIT;
+    float raw[NU][8], mag[NU];      // fp32 input: what is loaded, its largest magnitude
+    u32x4 raws[NU][2];              // split planes: what is loaded
+    unsigned hmax[NU], hmin[NU];    // and the extremes of its hi parts, pairwise
+    u32x4 sp[NU][2];
 #pragma unroll
-      for (int nb = 0; nb < NB; nb++) {
-        const float4 bq = xr[32 * nb * st];
-        acc[nb][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, bq.x, acc[nb][0], 0, 0, 0);
-        acc[nb][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, bq.y, acc[nb][0], 0, 0, 0);
-        acc[nb][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, bq.z, acc[nb][0], 0, 0, 0);
-        acc[nb][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, bq.w, acc[nb][0], 0, 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-        for (int cb = 0; cb < 2; cb++) {
-          const float2 bq = xr[(32 * nb + 16 * cb) * st];
-          acc[nb][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, bq.x, acc[nb][cb], 0, 0, 0);
-          acc[nb][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, bq.y, acc[nb][cb], 0, 0, 0);
-        }
+    for (int u = 0; u < NU; u++) {
+      mag[u] = 0.0f;
+      hmax[u] = hmin[u] = 0;
     }
-  };
-  auto tap = [&](const AT a, int k) {
-    if constexpr (RB == 32) mfma4(a, xs + lbase + k * dil);
-    else mfma4(a, xs2 + lbase + k * dil);
-  };
-  // The chunk loop, for a compile-time tap count KC (0: runtime K, A operands loaded per tap).
-  // Each chunk is straight-line code, so the scheduler can run LDS reads ahead of the MFMAs and
-  // count outstanding loads exactly: stage the window loaded one chunk earlier, issue the next
-  // chunk's window loads, then per tap four MFMAs on acur[k] followed by the load of that tap's
-  // operands for the next chunk into the same registers (prefetch distance about one chunk).  The
-  // last chunk is peeled so it issues no loads.
-  auto run = [&](auto kc, auto mask, auto nju) {
-    constexpr int KC = decltype(kc)::value;
-    constexpr int KA = KC > 0 ? KC : 1;
-    AT acur[KA];
-    auto chunk = [&](int j, auto with_loads) {
-      constexpr bool LD = decltype(with_loads)::value;
+    auto load_unit = [&](__amdgpu_buffer_rsrc_t rx, int u, int j) {
+      const int ci0 = (chunk0 + j) * CONV_CK;
+      if constexpr (SPLIT) {
+        const unsigned so = (unsigned) ci0 * ldx4;
+        raws[u][0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, voff[u], so, 0));
+        raws[u][1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, voff[u], so + 4u * ldx4, 0));
+        return;
+      }
+#pragma unroll
+      for (int r = 0; r < 8; r++) {
+        if constexpr (MASK) {   // a row past cin reads 0
+          const unsigned vo = voff[u] != PTK_OOB && ci0 + 8 * half + r < cin
+              ? voff[u] + (unsigned) (ci0 + r) * ldx4 : PTK_OOB;
+          raw[u][r] = buf_load(rx, vo, 0);
+        } else {
+          raw[u][r] = buf_load(rx, voff[u], (unsigned) (ci0 + r) * ldx4);
+        }
+      }
+    };
+    auto split_unit = [&](int u, int e) {   // channels 2e, 2e + 1 of this lane's eight
+      if constexpr (SPLIT) {
+        sp[u][0][e] = raws[u][0][e];
+        sp[u][1][e] = raws[u][1][e];
+        if (e & 1) {
+          asm("v_pk_maximum3_f16 %0, %1, %2, %0" : "+v"(hmax[u]) : "v"(raws[u][0][e - 1]), "v"(raws[u][0][e]));
+          asm("v_pk_minimum3_f16 %0, %1, %2, %0" : "+v"(hmin[u]) : "v"(raws[u][0][e - 1]), "v"(raws[u][0][e]));
+        }
+        return;
+      }
+      const float a = in_xform<IN>(raw[u][2 * e], in_a), b = in_xform<IN>(raw[u][2 * e + 1], in_a);
+      unsigned h, l;
+      mag[u] = max_mag(mag[u], a, b);
+      split_pair(a * (float) (1 << CONV_XS), b * (float) (1 << CONV_XS), h, l);
+      sp[u][0][e] = h;
+      sp[u][1][e] = l;
+    };
+    auto store_window = [&]() {
       __builtin_amdgcn_wave_barrier();
-      store_chunk((chunk0 + j) * CONV_CK, mask, nju);
+#pragma unroll
+      for (int u = 0; u < NU; u++)
+#pragma unroll
+        for (int q = 0; q < 2; q++) xs[half * PS + 2 * q * PS + 32 * u + l32] = sp[u][q];
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if constexpr (KC > 0) {
-        // the next chunk's window loads go out behind tap 0's MFMAs, not between the window
-        // store and the chunk's first MFMA
-#pragma unroll
-        for (int k = 0; k < KC; k++) {
-          tap(acur[k], k);
-          if constexpr (LD) {
-            if (k == 0) {
-              load_chunk((chunk0 + j + 1) * CONV_CK, mask, nju);
-              PTK_PIN_VMEM();
-            }
-            acur[k] = wa(k, j + 1);
-            PTK_PIN_VMEM();
-          }
-        }
-      } else {
-        if constexpr (LD) {
-          load_chunk((chunk0 + j + 1) * CONV_CK, mask, nju);
-          PTK_PIN_VMEM();
-        }
-        for (int k = 0; k < K; k++) tap(wa(k, j), k);
-      }
-      __builtin_amdgcn_wave_barrier();
     };
-    // window loads first, then the A operands: the same order as inside a chunk, so the wait
-    // before the first window store is the same count on entry as on every later trip
-    load_chunk(chunk0 * CONV_CK, mask, nju);
-    if constexpr (KC > 0) {
+    const int sc = KC > 0 ? 1 : st;   // the straight-line bodies take stride 1 only
+    const u32x4 *const xl = xs + half * PS + l32 * sc - dmin;   // tap 0, column block 0
+    auto col = [&](int k, int nb) {   // B operands of tap k, column block nb
+      const u32x4 *xr = xl + k * dil + 32 * nb * sc;
+      Parts q;
+      q.h = __builtin_bit_cast(f16x8, xr[0]);
+      q.l = __builtin_bit_cast(f16x8, xr[2 * PS]);
+      return q;
+    };
+    auto mfma3 = [&](const Parts &a, const Parts &c, int nb) {
+      acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.h, c.l, acc[nb], 0, 0, 0);
+      acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.l, c.h, acc[nb], 0, 0, 0);
+      acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.h, c.h, acc[nb], 0, 0, 0);
+    };
+    const __amdgpu_buffer_rsrc_t rx = x_rsrc(true), rw = w_rsrc(true);
+    const int last = nch * K - 1;   // the wave's last slice
+    Parts ahead[PD];
 #pragma unroll
-      for (int k = 0; k < KC; k++) acur[k] = wa(k, 0);
-    }
+    for (int u = 0; u < NU; u++) load_unit(rx, u, 0);
+#pragma unroll
+    for (int k = 0; k < PD; k++) ahead[k] = wa(rw, min(k, last));
     load_bias();
-    for (int j = 0; j + 1 < nch; j++) chunk(j, std::true_type{});
-    chunk(nch - 1, std::false_type{});
+    {
+      const __amdgpu_buffer_rsrc_t rx1 = x_rsrc(nch > 1);
+#pragma unroll
+      for (int u = 0; u < NU; u++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) split_unit(u, e);
+        load_unit(rx1, u, 1);
+      }
+    }
+    for (int j = 0; j < nch; j++) {
+      store_window();
+      const __amdgpu_buffer_rsrc_t rx2 = x_rsrc(j + 2 < nch);
+      if constexpr (KC > 0) {
+        // Steps of three MFMAs, (tap, column block).  A step's B operands are read while the step
+        // before it runs; the scheduling barrier keeps the compiler from reading further ahead,
+        // which would take more registers than there are.
+        constexpr int NS = KC * NB, S0 = NS / 3, NP = NU * 4;
+        Parts a[KC + PD];
+#pragma unroll
+        for (int k = 0; k < PD; k++) a[k] = ahead[k];
+        Parts q = col(0, 0);
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          const int k = s / NB, nb = s % NB;
+          Parts qn = q;
+          if (s + 1 < NS) qn = col((s + 1) / NB, (s + 1) % NB);
+          if (nb == 0) a[k + PD] = wa(rw, k + PD < KC ? j * KC + k + PD : min(j * KC + k + PD, last));
+          // the next chunk's split over the last two thirds of the steps
+#pragma unroll
+          for (int i = 0; i < NP; i++)
+            if (S0 + i * (NS - S0) / NP == s) {
+              split_unit(i / 4, i % 4);
+              if (i % 4 == 3) load_unit(rx2, i / 4, j + 2);
+            }
+          mfma3(a[k], q, nb);
+          __builtin_amdgcn_sched_barrier(0);
+          q = qn;
+        }
+#pragma unroll
+        for (int k = 0; k < PD; k++) ahead[k] = a[KC + k];
+      } else {
+        for (int k = 0; k < K; k++) {
+          const Parts a = ahead[0];
+          ahead[0] = wa(rw, min(j * K + k + 1, last));
+          PTK_PIN_VMEM();
+#pragma unroll
+          for (int nb = 0; nb < NB; nb++) mfma3(a, col(k, nb), nb);
+        }
+#pragma unroll
+        for (int u = 0; u < NU; u++) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) split_unit(u, e);
+          load_unit(rx2, u, j + 2);
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      if constexpr (SPLIT) {   // all zero alarms too: an input too small for hi and lo looks like that
+        const float m = max_mag(max_mag(0.0f, half_of(hmax[u], 0), half_of(hmax[u], 1)),
+                                half_of(hmin[u], 0), half_of(hmin[u], 1));
+        odd |= voff[u] != PTK_OOB && !(m <= 65504.0f && m >= 0.25f);
+      } else {
+        odd |= !conv_alarm_free(mag[u]);
+      }
+    }
+  };
+  // The second pass: the same chunks from fp32 operands, in one rolled loop.  The window is staged
+  // as planes [h][e >> 2] of float4 columns (channels 8h + e): the same LDS.
+  // the input transform as the fp32 operands need it: split planes hold LeakyReLU(in_a) of d.x
+  auto xform32 = [&](float v) {
+    return in_xform<IN == PTK_IN_PLAIN ? PTK_IN_PLAIN : PTK_IN_LEAKY>(v, in_a);
+  };
+  auto run32 = [&](const ptk_conv_desc &d) {
+    const int PS = g.wcols;
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        (void *) (d.x + xoff), (short) 0, (int) nrec, PTK_BUF_WORD3);
+    const float4 *const wr = reinterpret_cast<const float4 *>(d.w + (long long) (pi.mt * 32) * K * d.cinp) +
+                             ((long long) mb * nchunk + chunk0) * K * (CONV_TAPB / 16) + lane * 2;
+    float4 *const x4 = reinterpret_cast<float4 *>(xs);
+    for (int j = 0; j < nch; j++) {
+      const int ci0 = (chunk0 + j) * CONV_CK + 8 * half;
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int u = 0; u < CONV_NU_MAX; u++) {
+        if (32 * u >= PS) continue;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const unsigned c4 = IN == PTK_IN_SPLIT ? (voff[u] - (unsigned) (8 * half) * ldx4) / 4u
+                                                 : voff[u] - (unsigned) (8 * half) * ldx4;
+          v[e] = xform32(buf_load(rx, voff[u] != PTK_OOB && ci0 + e < cin
+                                          ? c4 + (unsigned) (ci0 + e) * ldx4 : PTK_OOB, 0));
+        }
+        x4[2 * half * PS + 32 * u + l32] = make_float4(v[0], v[1], v[2], v[3]);
+        x4[(2 * half + 1) * PS + 32 * u + l32] = make_float4(v[4], v[5], v[6], v[7]);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (int k = 0; k < K; k++) {
+        const float4 *const wk = wr + (long long) (j * K + k) * (CONV_TAPB / 16);
+        const float4 a0 = wk[0], a1 = wk[1];
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) {
+          const float4 *const xr = x4 + 2 * half * PS + (l32 + 32 * nb) * st - dmin + k * dil;
+          const float4 b0 = xr[0], b1 = xr[PS];
+          acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, b0.x, acc[nb], 0, 0, 0);
+          acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, b0.y, acc[nb], 0, 0, 0);
+          acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.z, b0.z, acc[nb], 0, 0, 0);
+          acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.w, b0.w, acc[nb], 0, 0, 0);
+          acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.x, b1.x, acc[nb], 0, 0, 0);
+          acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.y, b1.y, acc[nb], 0, 0, 0);
+          acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.z, b1.z, acc[nb], 0, 0, 0);
+          acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.w, b1.w, acc[nb], 0, 0, 0);
+        }
+      }
+    }
   };
   constexpr std::false_type nomask{};
-  constexpr std::integral_constant<int, 1> one{};
-  constexpr std::integral_constant<int, NJ> all{};
-  const bool narrow = XW <= 64;
-  if (cin == d.cinp) {
-    if constexpr (KT > 0) {
-      if (K == KT && narrow) run(std::integral_constant<int, KT>{}, nomask, one);
-      else if (K == KT) run(std::integral_constant<int, KT>{}, nomask, all);
-      else if (KT > 7 && K == 7 && narrow) run(std::integral_constant<int, 7>{}, nomask, one);
-      else if (KT > 3 && K == 3 && narrow) run(std::integral_constant<int, 3>{}, nomask, one);
-      else run(std::integral_constant<int, 0>{}, nomask, all);
-    } else {
-      run(std::integral_constant<int, 0>{}, nomask, all);
-    }
-  } else {
-    // channel padding in the last chunks: any K through the generic body
-    run(std::integral_constant<int, 0>{}, std::true_type{}, all);
-  }
+  constexpr std::integral_constant<int, NB + 1> few{};
+  constexpr std::integral_constant<int, CONV_NU_MAX> all{};
+  const bool narrow = XW <= 32 * (NB + 1);
+  // channel padding in the last chunk, a stride or another K: the rolled body
+  const int straight = cin == nchunk * CONV_CK && st == 1 ? K : 0;
+  if (nch == 0) load_bias();
+  else if (KT == 4 && straight == 4 && narrow) run(std::integral_constant<int, KT == 4 ? 4 : 0>{}, nomask, few);
+  else if (KT == 11 && straight == 11 && narrow) run(std::integral_constant<int, KT == 11 ? 11 : 0>{}, nomask, few);
+  else if (KT == 11 && straight == 11) run(std::integral_constant<int, KT == 11 ? 11 : 0>{}, nomask, all);
+  else if (KT == 11 && straight == 7 && narrow) run(std::integral_constant<int, KT == 11 ? 7 : 0>{}, nomask, few);
+  else if (KT == 11 && straight == 3 && narrow) run(std::integral_constant<int, KT == 11 ? 3 : 0>{}, nomask, few);
+  else run(std::integral_constant<int, 0>{}, std::true_type{}, all);
 
   // Epilogue: the S partial sums of a block are added in wave order through LDS, then bias, the
-  // epilogue chain and one store per output.  RB = 32: lane (l32, half) holds, for column block
-  // nb, the 16 values v of column q0 + 32*nb + l32 at rows 8*(v >> 2) + 4*half + (v & 3) of the
-  // block.  RB = 16: lane (l16, quad) holds 8 values v of column q0 + 32*nb + 16*(v >> 2) + l16 at
-  // rows 4*quad + (v & 3).  Wave ks of a column group finishes v in [v0, v0 + NV/S).
-  const long long qend = d.q0 + d.nq + (last_item ? d.ext_r : 0);
-  const int M = d.M, C4 = d.C4, ys = d.ys, ypad = d.ypad, nepi = d.nepi;
-  const long long Lout = d.Lout, ldy = d.ldy;
-  float *yb = d.y + (long long) b * d.bsy;
-  float *y2b = d.y2 != nullptr ? d.y2 + (long long) b * d.bsy : nullptr;
-  const float a2 = d.a2;
+  // epilogue chain and one store per output.  Lane (l32, half) holds, for column block nb, the 16
+  // values v of column q0 + 32*nb + l32 at rows 8*(v >> 2) + 4*half + (v & 3) of the block.  Wave w
+  // finishes the NMAX = 16 / S values from v0 = w * NMAX, in groups of GRP <= 4 (rows of one v >> 2).
+  constexpr int NMAX = 16 / S, GRP = NMAX < 4 ? NMAX : 4, NG = NMAX / GRP;
+  const int v0 = w * NMAX;
   const int addt = pi.addt;   // the chain's residual add, if any
-  const int nv = NV >> lgS, v0 = ks * nv, wg0 = cg * S;
-  // row and column of value v inside the block, lane parts included
-  auto vrow = [&](int v) { return RB == 32 ? 8 * (v >> 2) + 4 * half + (v & 3) : 4 * quad + (v & 3); };
-  auto vcol = [&](int nb, int v) { return RB == 32 ? 32 * nb + l32 : 32 * nb + 16 * (v >> 2) + l16; };
-
+  auto vrow = [&](int i) { return 8 * ((v0 + i) >> 2) + 4 * half + ((v0 + i) & 3); };   // of value i
+  unsigned mine = ~0u;   // bit nb: this pass stores the lane's column of block nb
+  bool again = false;    // some column is left to the second pass
+  for (int pass = 0;; pass++) {
+  // (an opaque copy of the problem index: the compiler would otherwise load everything the rare
+  // paths read ahead of the loop)
+  int pe = p;
+  asm volatile("" : "+s"(pe));
+  const ptk_conv_desc &d = g.d[pe];
   // Each wave writes its partial sums over its own staging area, which only it reads, so no wave
-  // waits for the others before writing (a separate region when they do not fit).
-  constexpr bool OWN_RED = Geo::OWN_RED;
-  auto red_of = [&](int wave) { return OWN_RED ? smem + wave * Geo::STG : smem + wave * Geo::RED; };
-  if constexpr (!OWN_RED) __syncthreads();
-  {
-    float *red = red_of(w);
+  // waits for the others before writing: [nb][v >> 2][lane] float4.
+  int *const flags = reinterpret_cast<int *>(smem + S * wslots);
+  if constexpr (S > 1) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    f32x4 *red = reinterpret_cast<f32x4 *>(xs);
 #pragma unroll
     for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-      for (int cb = 0; cb < NCB; cb++)
+      for (int q = 0; q < 4; q++) {
+        f32x4 v;
 #pragma unroll
-        for (int v = 0; v < NV / NCB; v++) red[(nb * NV + cb * (NV / NCB) + v) * 64 + lane] = acc[nb][cb][v];
+        for (int i = 0; i < 4; i++) v[i] = acc[nb][4 * q + i];
+        red[(nb * 4 + q) * 64 + lane] = v;
+      }
   }
+  const bool alarm = pass == 0 && __ballot(odd || scale_r != scale_r) != 0;
+  if (S > 1 && pass == 0 && lane == 0) flags[w] = alarm;
+  // the barrier behind the partial sums; then, in a workgroup that was alarmed, the columns that
+  // are left to the second pass
   auto reduce_wait = [&]() {
-    if (S > 1) {
-      __syncthreads();
-    } else {   // S = 1: a wave reads back only what it wrote
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if constexpr (S > 1) __syncthreads();
+    if (pass != 0) return;
+    int any = alarm;
+    if constexpr (S > 1) {
+#pragma unroll
+      for (int i = 0; i < S; i++) any |= flags[i];
     }
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(any) == 0, 1)) return;
+    float *const cm = reinterpret_cast<float *>(smem + S * wslots + 2);   // per window column
+    for (int i = threadIdx.x; i < XW; i += 64 * S) {
+      const int c = cmin + i, pc = pi.flags & PROB_REFLECT ? (c == 0 ? 1 : c - 1) : c;
+      float m = 0.0f;
+      if (c >= 0 && c < lim)
+        for (int ci = 0; ci < cin; ci++) m = max_mag(m, xform32(d.x[xoff + (long long) ci * d.ldx + pc]), 0.0f);
+      cm[i] = m;
+    }
+    __syncthreads();
+    const bool bad_w = __ballot(scale_r != scale_r) != 0;
+    const long long qend = d.q0 + d.nq + (last_item ? d.ext_r : 0);
+    mine = 0;
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) {
+      float m = 0.0f;
+      for (int k = 0; k < K; k++) m = max_mag(m, cm[(l32 + 32 * nb) * st - dmin + k * dil], 0.0f);
+      // (a column past the end is stored by neither pass)
+      if (q0 + 32 * nb + l32 >= qend || (!bad_w && conv_fits(m))) mine |= 1u << nb;
+    }
+    again = __ballot(mine != (1u << NB) - 1) != 0;
   };
-  // The S partial sums of a value in wave order.  Every read is issued (a wave past the split
-  // re-reads the group's first, in bounds, and is not added), so the reads of all values go out
-  // together behind one wait instead of one round trip each behind a branch.
-  auto reduced = [&](int nb, int v) {
-    const int o = (nb * NV + v) * 64 + lane;
-    float part[NW];
+  // The S partial sums of GRP values in wave order.
+  auto reduced = [&](int nb, int gg, float *val) {
+    if constexpr (S > 1) {
+      const int v = v0 + gg * GRP;
+      typedef float vec __attribute__((ext_vector_type(GRP)));
+      vec part[S];
 #pragma unroll
-    for (int i = 0; i < NW; i++) part[i] = red_of(wg0 + (i < S ? i : 0))[o];
-    float sum = part[0];
+      for (int i = 0; i < S; i++)
+        part[i] = *reinterpret_cast<const vec *>(reinterpret_cast<const float *>(smem + i * wslots) +
+                                                 (((nb * 4 + (v >> 2)) * 64 + lane) * 4 + (v & 3)));
+      vec sum = part[0];
 #pragma unroll
-    for (int i = 1; i < NW; i++) sum = i < S ? sum + part[i] : sum;
-    return sum;
+      for (int i = 1; i < S; i++) sum += part[i];
+#pragma unroll
+      for (int i = 0; i < GRP; i++) val[gg * GRP + i] = sum[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < GRP; i++) val[gg * GRP + i] = acc[nb][gg * GRP + i];
+    }
   };
   // Fast path: a full block whose rows are consecutive output channels (conv, or a convT block
   // inside one phase), with every index of the output, its LeakyReLU copy and the residual inside
   // 32 bits (the launcher checks the extents).  Addresses are a wave-uniform row offset, in the
   // scalar offset of a buffer access, plus a lane offset computed once per column; the residual
   // loads are issued before the reduction barrier, at a clamped column so that every lane loads
-  // in bounds without a branch (a lane whose column does not exist stores nothing).  The values
-  // of a lane are val[i], i < nv: value v0 + i of the block.  The chain runs op by op over all of
-  // them, one branch per op.  A convT block with its rows interleaved by phase (phase_il) holds
-  // RB / 4 whole channels; its stores are laid out below.
-  if ((pi.flags & PROB_FAST) && (one_phase || phase_il) && mb * RB + RB <= pi.M) {
-    const ConvEpi ep = g.ep[p];
-    // a wave finishes at most NMAX values (NV over the smallest split of its workgroup size),
-    // in groups of GRP that share a column block (nv is a multiple of GRP)
-    constexpr int NMAX = NW == 8 ? NV / 8 : NV;
-    constexpr int GRP = (RB == 32 ? 4 : 2) < NMAX ? (RB == 32 ? 4 : 2) : NMAX, NG = NMAX / GRP;
-    const int ngrp = nv / GRP;
+  // in bounds without a branch (a lane whose column does not exist stores nothing).  The chain runs
+  // op by op over a lane's values, one branch per op.  A convT block with its rows interleaved by
+  // phase (phase_il) holds 8 whole channels.
+  if ((pi.flags & PROB_FAST) && (one_phase || phase_il) && mb * 32 + 32 <= pi.M) {
+    const ConvEpi ep = g.ep[pe];
     // first channel of the block
-    const long long row0 = phase_il ? (long long) mb * (RB / 4) : (long long) mb * RB - (long long) r_tile * ep.C4;
+    const long long row0 = phase_il ? (long long) mb * 8 : (long long) mb * 32 - (long long) r_tile * ep.C4;
     const int ldy32 = ep.ldy, ldt32 = ep.ldt;
     float *yk = const_cast<float *>(ep.y) + (long long) b * ep.bsy + row0 * ldy32;
     const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(
@@ -1014,200 +1177,163 @@ __global__ void __launch_bounds__(64 * NW) conv_mfma_kernel(const ConvGroup g) {
     const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(
         (void *) (addt >= 0 ? ep.t + (long long) b * ep.bst + row0 * ldt32 : yk), (short) 0,
         (int) 0x7fffffff, PTK_BUF_WORD3);
-    // lane part of the row of value i, and its wave-uniform part
-    const int lrow = RB == 32 ? 4 * half : 4 * quad;
-    auto urow = [&](int i) { return RB == 32 ? 8 * (((v0 + i) >> 2)) + ((v0 + i) & 3) : ((v0 + i) & 3); };
+    const __amdgpu_buffer_rsrc_t rys = __builtin_amdgcn_make_buffer_rsrc(
+        (void *) (ep.ysp != nullptr ? reinterpret_cast<const float *>(ep.ysp) + (long long) b * ep.bsy + row0 * ldy32 : yk),
+        (short) 0, (int) 0x7fffffff, PTK_BUF_WORD3);
+    // wave-uniform part of the row of value i (the lane part is 4 * half)
+    auto urow = [&](int i) { return 8 * ((v0 + i) >> 2) + ((v0 + i) & 3); };
     const int qend32 = ep.qend + (last_item ? ep.ext_r : 0);
+    float rv[NB][NMAX];
+    if (addt >= 0) {
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) {
+        const int q = q0 + 32 * nb + l32;
+        const int col = q * ep.ys + r_tile - ep.ypad;
+        const int cl = q < qend32 && col >= 0 && col < ep.lout ? col : 0;
+#pragma unroll
+        for (int i = 0; i < NMAX; i++)
+          rv[nb][i] = buf_load(rt, (unsigned) (4 * half * ldt32 + cl) * 4u, (unsigned) (urow(i) * ldt32) * 4u);
+      }
+    }
+    reduce_wait();
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
-      // columns of this lane: one per column block (RB = 32), two (RB = 16)
-      bool ok[NCB], oq[NCB];
-      int cl[NCB], cu[NCB];
+      const int q = q0 + 32 * nb + l32;
+      const int col = q * ep.ys + r_tile - ep.ypad;   // phase_il: the sample of phase 0 (r_tile = 0)
+      const bool oq = q < qend32 && (mine >> nb & 1);
+      float val[NMAX];
 #pragma unroll
-      for (int cb = 0; cb < NCB; cb++) {
-        const int q = (int) q0 + 32 * nb + (RB == 32 ? l32 : 16 * cb + l16);
-        const int col = q * ep.ys + r_tile - ep.ypad;
-        oq[cb] = q < qend32;
-        cu[cb] = col;   // phase_il: the sample of phase 0 (r_tile = 0), unclamped
-        ok[cb] = oq[cb] && col >= 0 && col < ep.lout;
-        cl[cb] = ok[cb] ? col : 0;
-      }
-      auto cbo = [&](int i) { return RB == 32 ? 0 : ((v0 + i) >> 2); };
-      // column / test of column block c as a select (an index into cl / ok that is not a
-      // compile-time constant would put the arrays in scratch memory)
-      auto clof = [&](int c) { return NCB == 1 || c == 0 ? cl[0] : cl[NCB - 1]; };
-      auto okof = [&](int c) { return NCB == 1 || c == 0 ? ok[0] : ok[NCB - 1]; };
-      float rv[NMAX], val[NMAX];
-      if (addt >= 0) {
+      for (int gg = 0; gg < NG; gg++) reduced(nb, gg, val);
 #pragma unroll
-        for (int gg = 0; gg < NG; gg++)
-          if (gg < ngrp)
+      for (int i = 0; i < NMAX; i++)
+        val[i] = __fadd_rn(bias_of(4 * half + urow(i)), val[i] * scale_of(4 * half + urow(i)));
+      // The chain.  The decoder's two chains, a LeakyReLU and a tensor add (the chain's one, the
+      // launcher's rule), have their own code; any other goes op by op.
+      if (ep.ops == PTK_EPI_ADDT) {
 #pragma unroll
-            for (int jj = 0, i = gg * GRP; jj < GRP; jj++, i++)
-            rv[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                rt, (unsigned) (lrow * ldt32 + clof(cbo(i))) * 4u, (unsigned) (urow(i) * ldt32) * 4u, 0));
-      }
+        for (int i = 0; i < NMAX; i++) val[i] = val[i] + rv[nb][i];
+      } else if (ep.ops == PTK_EPI_LEAKY) {
 #pragma unroll
-      for (int gg = 0; gg < NG; gg++)
-        if (gg < ngrp)
+        for (int i = 0; i < NMAX; i++) val[i] = val[i] >= 0.0f ? val[i] : ep.a[0] * val[i];
+      } else {
+#pragma unroll 1
+        for (int e = 0; e < ep.nepi; e++) {
+          const int op = (ep.ops >> (4 * e)) & 15;
+          const float a = e == 0 ? ep.a[0] : e == 1 ? ep.a[1] : e == 2 ? ep.a[2] : ep.a[3];
 #pragma unroll
-          for (int jj = 0, i = gg * GRP; jj < GRP; jj++, i++) val[i] = bias_of(lrow + urow(i));
-      if (nb == 0) reduce_wait();
-#pragma unroll
-      for (int gg = 0; gg < NG; gg++)
-        if (gg < ngrp)
-#pragma unroll
-          for (int jj = 0, i = gg * GRP; jj < GRP; jj++, i++) val[i] += reduced(nb, v0 + i);
-      // the chain op by op over the four slots (straight-line: a rolled loop over the ops made the
-      // compiler copy the value array at every op); a slot past nepi is skipped by a uniform branch
-#pragma unroll
-      for (int e = 0; e < PTK_MAX_EPI; e++) {
-        if (e >= ep.nepi) break;
-        const int op = (ep.ops >> (4 * e)) & 15;
-        const float a = ep.a[e];
-        if (op == PTK_EPI_LEAKY) {
-#pragma unroll
-          for (int gg = 0; gg < NG; gg++)
-            if (gg < ngrp)
-#pragma unroll
-              for (int jj = 0, i = gg * GRP; jj < GRP; jj++, i++) val[i] = val[i] >= 0.0f ? val[i] : a * val[i];
-        } else if (op == PTK_EPI_RELU) {
-#pragma unroll
-          for (int gg = 0; gg < NG; gg++)
-            if (gg < ngrp)
-#pragma unroll
-              for (int jj = 0, i = gg * GRP; jj < GRP; jj++, i++) val[i] = val[i] > 0.0f ? val[i] : 0.0f;
-        } else if (op == PTK_EPI_MULS) {
-#pragma unroll
-          for (int gg = 0; gg < NG; gg++)
-            if (gg < ngrp)
-#pragma unroll
-              for (int jj = 0, i = gg * GRP; jj < GRP; jj++, i++) val[i] = val[i] * a;
-        } else if (op == PTK_EPI_ADDS) {
-#pragma unroll
-          for (int gg = 0; gg < NG; gg++)
-            if (gg < ngrp)
-#pragma unroll
-              for (int jj = 0, i = gg * GRP; jj < GRP; jj++, i++) val[i] = val[i] + a;
-        } else if (op == PTK_EPI_DIVS) {
-#pragma unroll
-          for (int gg = 0; gg < NG; gg++)
-            if (gg < ngrp)
-#pragma unroll
-              for (int jj = 0, i = gg * GRP; jj < GRP; jj++, i++) val[i] = val[i] / a;
-        } else if (op == PTK_EPI_ADDT) {   // the chain's one tensor add (the launcher's rule)
-#pragma unroll
-          for (int gg = 0; gg < NG; gg++)
-            if (gg < ngrp)
-#pragma unroll
-              for (int jj = 0, i = gg * GRP; jj < GRP; jj++, i++) val[i] = val[i] + rv[i];
-        }
-      }
-      if (phase_il) {
-        // Rows interleaved by phase: the GRP values of a group are consecutive phases p0 .. of one
-        // channel at one column (RB = 32: channel 2 * (v >> 2) + half of the block; RB = 16:
-        // channel quad, column block v >> 2), so they go to GRP consecutive samples.  Stored in
-        // pairs, 8 bytes from one lane, where both samples exist; one by one at the sequence
-        // ends.  Every address is formed from an existing sample (0 otherwise).
-        const int chl = RB == 32 ? half : quad;
-        auto cuof = [&](int c) { return NCB == 1 || c == 0 ? cu[0] : cu[NCB - 1]; };
-        auto oqof = [&](int c) { return NCB == 1 || c == 0 ? oq[0] : oq[NCB - 1]; };
-        typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-#pragma unroll
-        for (int gg = 0; gg < NG; gg++)
-          if (gg < ngrp) {
-            const int vg = v0 + gg * GRP, cb = cbo(gg * GRP);
-            const unsigned so = (unsigned) ((RB == 32 ? 2 * (vg >> 2) : 0) * ldy32) * 4u;
-            const bool inq = oqof(cb);
-            if constexpr (GRP == 1) {   // one value per wave (16-row tiles, 8-way split)
-              const int sa = cuof(cb) + (vg & 3);
-              if (inq && sa >= 0 && sa < ep.lout) {
-                const unsigned vo = (unsigned) (chl * ldy32 + sa) * 4u;
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(val[gg]), ry, vo, so, 0);
-                if (ep.y2 != nullptr)
-                  __builtin_amdgcn_raw_buffer_store_b32(
-                      __float_as_uint(val[gg] >= 0.0f ? val[gg] : ep.a2 * val[gg]), ry2, vo, so, 0);
-              }
-              continue;
-            }
-#pragma unroll
-            for (int jj = 0; jj < GRP; jj += 2) {
-              const int i = gg * GRP + jj;
-              const int sa = cuof(cb) + (vg & 3) + jj;   // sample of value i; value i + 1 at sa + 1
-              const bool va = inq && sa >= 0 && sa < ep.lout;
-              const bool vb = inq && sa + 1 >= 0 && sa + 1 < ep.lout;
-              const int sb = va ? sa : (vb ? sa + 1 : 0);
-              const unsigned vo = (unsigned) (chl * ldy32 + sb) * 4u;
-              const float y2a = val[i] >= 0.0f ? val[i] : ep.a2 * val[i];
-              const float y2b = val[i + 1] >= 0.0f ? val[i + 1] : ep.a2 * val[i + 1];
-              if (va && vb) {
-                __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(val[i]), __float_as_uint(val[i + 1])}, ry, vo, so, 0);
-                if (ep.y2 != nullptr)
-                  __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(y2a), __float_as_uint(y2b)}, ry2, vo, so, 0);
-              } else if (va || vb) {
-                const float one = va ? val[i] : val[i + 1];
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(one), ry, vo, so, 0);
-                if (ep.y2 != nullptr)
-                  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(va ? y2a : y2b), ry2, vo, so, 0);
-              }
-            }
-          }
-        continue;
-      }
-      // a group shares its column block, so one test covers its stores
-#pragma unroll
-      for (int gg = 0; gg < NG; gg++)
-        if (gg < ngrp && okof(cbo(gg * GRP))) {
-          const unsigned vo = (unsigned) (lrow * ldy32 + clof(cbo(gg * GRP))) * 4u;
-#pragma unroll
-          for (int jj = 0, i = gg * GRP; jj < GRP; jj++, i++) {
-            const unsigned so = (unsigned) (urow(i) * ldy32) * 4u;
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(val[i]), ry, vo, so, 0);
-            if (ep.y2 != nullptr)
-              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(val[i] >= 0.0f ? val[i] : ep.a2 * val[i]), ry2, vo, so, 0);
+          for (int i = 0; i < NMAX; i++) {
+            const float v = val[i];
+            val[i] = op == PTK_EPI_LEAKY ? (v >= 0.0f ? v : a * v) : op == PTK_EPI_RELU ? (v > 0.0f ? v : 0.0f)
+                   : op == PTK_EPI_MULS ? v * a : op == PTK_EPI_ADDS ? v + a : op == PTK_EPI_DIVS ? v / a
+                   : op == PTK_EPI_ADDT ? v + rv[nb][i] : v;
           }
         }
+      }
+      // Stores by groups: four (or two) rows of one v >> 2.  Rows interleaved by phase: v >> 2 is
+      // the phase, the column's sample.
+#pragma unroll
+      for (int gg = 0; gg < NG; gg++) {
+        const int vg = v0 + gg * GRP;
+        const int cg = phase_il ? col + (vg >> 2) : col;
+        const int rg = phase_il ? (vg & 3) : urow(gg * GRP);   // uniform part of the group's first row
+        if (!(oq && cg >= 0 && cg < ep.lout)) continue;
+        const unsigned vo = (unsigned) (4 * half * ldy32 + cg) * 4u;
+#pragma unroll
+        for (int i = 0; i < GRP; i++) {
+          const float v = val[gg * GRP + i];
+          const unsigned so = (unsigned) ((rg + i) * ldy32) * 4u;
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ry, vo, so, 0);
+          if (ep.y2 != nullptr)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v >= 0.0f ? v : ep.a2 * v), ry2, vo, so, 0);
+        }
+        if (ep.ysp != nullptr) {
+          // channel 4 * half + (rg & 3) of the eight-channel group rg >> 3, hi row then lo row
+          unsigned h[GRP / 2], l[GRP / 2];
+#pragma unroll
+          for (int i = 0; i < GRP; i += 2) {
+            const float a = val[gg * GRP + i], c = val[gg * GRP + i + 1];
+            split_pair((a >= 0.0f ? a : ep.a2 * a) * (float) (1 << CONV_XS),
+                       (c >= 0.0f ? c : ep.a2 * c) * (float) (1 << CONV_XS), h[i / 2], l[i / 2]);
+          }
+          const unsigned vs = (unsigned) cg * 16u + (unsigned) half * 8u;
+          const unsigned ss = (unsigned) ((rg >> 3) * 8 * ldy32) * 4u + (unsigned) (rg & 3) * 2u;
+          if constexpr (GRP == 4) {
+            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64(u32x2{h[0], h[1]}, rys, vs, ss, 0);
+            __builtin_amdgcn_raw_buffer_store_b64(u32x2{l[0], l[1]}, rys, vs, ss + 16u * (unsigned) ldy32, 0);
+          } else {
+            __builtin_amdgcn_raw_buffer_store_b32(h[0], rys, vs, ss, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(l[0], rys, vs, ss + 16u * (unsigned) ldy32, 0);
+          }
+        }
+      }
     }
-    return;
-  }
-
+  } else {
   // General path (partial row blocks, convT phases that straddle a block, large tensors): per
   // element
+  const int M = d.M, C4 = d.C4, ys = d.ys, ypad = d.ypad, nepi = d.nepi;
+  const long long Lout = d.Lout, ldy = d.ldy;
+  float *yb = d.y + (long long) b * d.bsy;
+  float *y2b = d.y2 != nullptr ? d.y2 + (long long) b * d.bsy : nullptr;
+  float *ysb = d.ysp != nullptr ? reinterpret_cast<float *>(d.ysp) + (long long) b * d.bsy : nullptr;
+  const float a2 = d.a2;
+  const bool phase_rows = C4 != M;
+  const long long qend = d.q0 + d.nq + (last_item ? d.ext_r : 0);
   reduce_wait();
-  auto emit = [&](int nb, int v, float sum) {
-    const int m = mb * RB + vrow(v);
-    const long long q = q0 + vcol(nb, v);
-    if (m >= M || q >= qend) return;
-    int co = m, r = 0;
-    if (phase_il) {
-      r = m & 3;
-      co = m >> 2;
-    } else if (phase_rows) {
-      r = m / C4;
-      co = m - r * C4;
+#pragma unroll
+  for (int nb = 0; nb < NB; nb++) {
+    const long long q = (long long) q0 + 32 * nb + l32;
+    float val[NMAX];
+#pragma unroll
+    for (int gg = 0; gg < NG; gg++) reduced(nb, gg, val);
+#pragma unroll
+    for (int i = 0; i < NMAX; i++) {
+      const int m = mb * 32 + vrow(i);
+      float v = __fadd_rn(bias_of(vrow(i)), val[i] * scale_of(vrow(i)));   // all lanes active here
+      if (m >= M || q >= qend || !(mine >> nb & 1)) continue;
+      int co = m, r = 0;
+      if (phase_il) {
+        r = (m >> 3) & 3;
+        co = (m >> 5) * 8 + (m & 7);
+      } else if (phase_rows) {
+        r = m / C4;
+        co = m - r * C4;
+      }
+      const long long col = q * ys + r - ypad;
+      if (col < 0 || col >= Lout) continue;
+      for (int e = 0; e < nepi; e++) v = epi_apply(v, d.epi[e], b, co, col);
+      const long long yi = (long long) co * ldy + col;
+      yb[yi] = v;
+      const float vl = v >= 0.0f ? v : a2 * v;
+      if (y2b != nullptr) y2b[yi] = vl;
+      if (ysb != nullptr) {
+        unsigned h, l;
+        split_pair(vl * (float) (1 << CONV_XS), 0.0f, h, l);
+        unsigned short *const ys16 = reinterpret_cast<unsigned short *>(ysb + (long long) (co & ~7) * ldy) + col * 8 + (co & 7);
+        ys16[0] = (unsigned short) h;
+        ys16[8 * ldy] = (unsigned short) l;
+      }
     }
-    const long long col = q * ys + r - ypad;
-    if (col < 0 || col >= Lout) return;
-    float val = sum;
-    for (int e = 0; e < nepi; e++) val = epi_apply(val, d.epi[e], b, co, col);
-    const long long yi = (long long) co * ldy + col;
-    yb[yi] = val;
-    if (y2b != nullptr) y2b[yi] = val >= 0.0f ? val : a2 * val;
-  };
+  }
+  }
+  if (__builtin_expect(!again, 1)) break;
+  // the columns left over, from fp32 operands
+  again = false;
+  mine = ~mine;
+  scale_r = 1.0f;
 #pragma unroll
   for (int nb = 0; nb < NB; nb++)
-    for (int vv = 0; vv < nv; vv++) {
-      const int v = v0 + vv;
-      const float bv = bias_of(vrow(v));   // all lanes active here
-      emit(nb, v, reduced(nb, v) + bv);
-    }
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[nb][v] = 0.0f;
+  __syncthreads();   // every wave is done with the first pass's partial sums
+  if (nch > 0) run32(d);
+  }
 }
 
 static int conv_window(const ptk_conv_desc *d, int nb) {
   const int kd = (d->K - 1) * d->dil;
   return (32 * nb - 1) * d->stride + (kd < 0 ? -kd : kd) + 1;
 }
-static int win_max(int nb) { return nb == 2 ? WinGeo<2>::XWMAX : WinGeo<1>::XWMAX; }
 
 // Kernel-selection knobs (PTK_*), read from the environment once per process, at the first
 // launch that consults them, not per launch: launches come from many serving threads at once, and
@@ -1215,14 +1341,13 @@ static int win_max(int nb) { return nb == 2 ? WinGeo<2>::XWMAX : WinGeo<1>::XWMA
 // (tests that change a knob between calls); each is an atomic int, so a launch running meanwhile
 // sees the old or the new value of each knob.
 enum KnobId {
-  KN_CONV_SPLIT, KN_CONV_RB, KN_CONV_S8, KN_CONV_S8_MAX, KN_CONV_NB, KN_CONV_FAST, KN_TAIL_OUT,
+  KN_CONV_SPLIT, KN_CONV_NB, KN_CONV_FAST, KN_TAIL_OUT,
   KN_TAIL_GRID, KN_TAIL_XCD, KN_NARROW, KN_COUNT
 };
 static const struct {
   const char *name;
   int dflt;
-} kKnobs[KN_COUNT] = {{"PTK_CONV_SPLIT", 0}, {"PTK_CONV_RB", 0},    {"PTK_CONV_S8", 1},
-                      {"PTK_CONV_S8_MAX", 1536}, {"PTK_CONV_NB", 0}, {"PTK_CONV_FAST", 1},
+} kKnobs[KN_COUNT] = {{"PTK_CONV_SPLIT", 0}, {"PTK_CONV_NB", 0}, {"PTK_CONV_FAST", 1},
                       {"PTK_TAIL_OUT", 0},
                       {"PTK_TAIL_GRID", 0},   {"PTK_TAIL_XCD", 1},  {"PTK_NARROW", 1}};
 static std::atomic<int> g_knob[KN_COUNT];
@@ -1245,128 +1370,49 @@ extern "C" void ptk_knobs_reload(void) {
   knobs_read();
 }
 
-// Tile shape (RB rows, channel split S in {1, 2, 4, 8}; PTK_CONV_RB and PTK_CONV_SPLIT override).
-// All waves of a launch usually fit on the chip at once, so a launch lasts as long as its busiest
-// SIMD: with W waves over the 1024 SIMDs (256 CUs x 4) that SIMD holds ceil(W / 1024) of them
-// while the mean is W / 1024.  Fewer than ~3 waves per SIMD also leave MFMA latency exposed (a
-// lone wave keeps its SIMD's matrix pipe ~60 % busy), and each split step costs its LDS reduction
-// and a share of the edges.  The model below, fitted to decoder shapes measured on MI355X (batch 1
-// and 22, C 128 / 256, K 3-11), picks the shape with the best predicted MFMA occupancy:
-//   eff = [mean / max waves per SIMD] x [latency hiding at the mean] x [split cost]
-//         x [rows that exist / rows computed] x [16-row tile cost]
-// evaluated on ONE batch item's grid (of nq_shape columns when the launch covers a sub-range).
-// The shape fixes the order in which a block's partial sums are added, so choosing it without the
-// batch size makes a batched item's result bit-identical to the same item decoded alone (and it
-// measured faster at batch 8 than a batch-aware choice).
-// 16-row tiles double the waves of a grid (and cut the padding of row counts like 72), at twice
-// the window staging and epilogue work per MFMA.  They need the 16-row weight copy (w16) and are
-// offered to single-problem launches only (PTK_CONV_RB=16 forces them on any launch with the
-// copy): the grouped MRF launches at small T ran as fast or faster alone on 16-row tiles, but
-// the concurrent serving step, where other streams fill the chip anyway, lost 1.4 % of its
-// throughput to their extra work per MFMA.  kRb16Cost = 0.7 puts conv_pre (T 226) and conv_post
-// on 16-row tiles and keeps ups.0 / ups.1 on 32-row ones, as measured at batch 1.
-static const double kSimds = 1024.0;
-static const double kRb16Cost = 0.70;
-static double split_eff(long long waves, int S) {
-  const double m = (double) waves / kSimds;
-  // past residency the extra waves run as one more wave on the SIMDs they land on
-  const double busiest = ceil(m);
-  const double balance = m / (busiest > 0.0 ? busiest : 1.0);
-  const double mh = m < 4.0 ? m : 4.0;
-  const double hide = mh >= 2.75 ? 1.0 : 0.45 + 0.2 * mh;
-  const double cost = S == 1 ? 1.0 : (S == 2 ? 0.97 : 0.90);
-  return balance * hide * cost;
-}
-static int choose_tiles(const ptk_conv_desc *const *ds, int n, int nb, int *rb_out) {
-  const int env_s = knob(KN_CONV_SPLIT), env_rb = knob(KN_CONV_RB);
-  bool rb16_ok = nb == 1 && (n == 1 || env_rb == 16);
-  for (int i = 0; i < n; i++)
-    if (ds[i]->w16 == nullptr) rb16_ok = false;
-  int best = 4, best_rb = 32;
-  long long best_waves = 0;
-  double best_eff = -1.0;
-  for (int RB = 32; RB >= 16; RB /= 2) {
-    if (RB == 16 && !rb16_ok) continue;
-    if ((env_rb == 16 || env_rb == 32) && RB != env_rb && (env_rb == 32 || rb16_ok)) continue;
-    for (int S = 1; S <= 4; S *= 2) {
-      if ((env_s == 1 || env_s == 2 || env_s == 4) && S != env_s) continue;
-      const int G = 4 / S;
-      long long waves = 0;
-      double rows = 0.0, rows_run = 0.0;
-      for (int i = 0; i < n; i++) {
-        const ptk_conv_desc *d = ds[i];
-        const long long nq = d->nq_shape > 0 ? d->nq_shape : d->nq;
-        const long long mt = (d->M + RB - 1) / RB;
-        const long long tiles = mt * ((nq + 32LL * nb * G - 1) / (32LL * nb * G));
-        waves += 4LL * tiles;
-        const double work = (double) nq * d->K * d->cinp;
-        rows += work * d->M;
-        rows_run += work * (double) (mt * RB);
-      }
-      const double e = split_eff(waves, S) * (rows_run > 0.0 ? rows / rows_run : 1.0) *
-                       (RB == 16 ? kRb16Cost : 1.0);
-      if (e > best_eff + 1e-9) {
-        best_eff = e;
-        best = S;
-        best_rb = RB;
-        best_waves = waves;
-      }
-    }
+// Tile shape: the channel split S in {2, 4} (PTK_CONV_SPLIT overrides) and the column blocks per
+// wave NB in {1, 2} (PTK_CONV_NB).
+// S fixes the order in which a block's partial sums are added, so it is chosen from one batch item's
+// grid (of nq_shape columns when the launch covers a sub-range): a batched item's result is
+// bit-identical to the same item alone.  NB changes no bit and is chosen from the whole launch.
+static void choose_tiles(const ptk_conv_desc *const *ds, int n, int *S_out, int *nb_out) {
+  const int env_s = knob(KN_CONV_SPLIT), env_nb = knob(KN_CONV_NB);
+  bool nb2_ok = true;
+  long long wgs = 0, item = 0;
+  for (int i = 0; i < n; i++) {
+    const ptk_conv_desc *d = ds[i];
+    if (conv_window(d, 2) > 32 * CONV_NU_MAX) nb2_ok = false;
+    const long long mt = (d->M + 31) / 32, nq = d->nq_shape > 0 ? d->nq_shape : d->nq;
+    wgs += d->batch * mt * ((d->nq + 63) / 64);
+    item += mt * ((nq + 63) / 64);
   }
-  // The 8-way split (8-wave workgroups over the same tiles): for a single problem on 32-row
-  // tiles whose 4-way grid leaves one lone wave on most SIMDs (1 to 1.5 waves per SIMD), it
-  // doubles the waves that hide each other's latency at the cost of twice the partial sums.  On
-  // 16-row tiles, which already do more staging and epilogue work per MFMA, it measured no faster
-  // alone and slower batched.  Needs whole chunks for all eight waves (cinp a multiple of 64).
-  // PTK_CONV_SPLIT=8 forces it where it applies, PTK_CONV_S8=0 turns the rule off,
-  // PTK_CONV_S8_MAX sets the upper bound in waves (1536).
-  const bool s8_ok = nb == 1 && n == 1 && ds[0]->cinp % (8 * CONV_CK) == 0;
-  const long long s8_max = knob(KN_CONV_S8_MAX);
-  if (s8_ok && (env_s == 8 || (env_s == 0 && knob(KN_CONV_S8) != 0 && best == 4 &&
-                               best_rb == 32 && best_waves >= (long long) kSimds &&
-                               best_waves < s8_max)))
-    best = 8;
-  *rb_out = best_rb;
-  return best;
-}
-
-// column blocks per wave: 1.  Two blocks halve the weight loads per MFMA but double the window
-// registers and halve the grid; on MI355X they lost at every decoder shape measured (batch 1 and
-// 8), so they are only used when PTK_CONV_NB=2 asks for them.
-static int choose_nb(const ptk_conv_desc *d) {
-  const int env_nb = knob(KN_CONV_NB);
-  if (env_nb == 2 && conv_window(d, 2) <= win_max(2)) return 2;
-  return 1;
+  *nb_out = nb2_ok && (env_nb == 2 || (env_nb != 1 && wgs >= 200)) ? 2 : 1;
+  *S_out = env_s == 2 || env_s == 4 ? env_s : item >= 640 ? 2 : 4;
 }
 
 extern "C" int ptk_conv_mfma_ok(const ptk_conv_desc *d) {
   if (d->M < 16 || d->cin < 2 || d->K < 1 || d->stride < 1 || d->dil == 0) return 0;
-  if (conv_window(d, 1) > win_max(1)) return 0;
+  if (conv_window(d, 1) > 32 * CONV_NU_MAX) return 0;
   if (d->cinp != ptk_conv_cinp(d->cin)) return 0;
   // 32-bit buffer offsets: every row offset plus the out-of-range marker must stay below 2^32
   if ((unsigned long long) d->cinp * (unsigned long long) d->ldx * 4ULL >= 0x80000000ULL) return 0;
   return 1;
 }
 
-template <int KT, int NB, int IN, int RB, int NW>
-static void launch_conv(const ConvGroup &g, dim3 grid, hipStream_t s) {
-  constexpr size_t lds = LdsGeo<NB, RB, NW>::BYTES;
-  hipLaunchKernelGGL((conv_mfma_kernel<KT, NB, IN, RB, NW>), grid, dim3(64 * NW), lds, s, g);
+template <int KT, int NB, int IN>
+static void launch_conv_s(int S, const ConvGroup &g, dim3 grid, hipStream_t s) {
+  const size_t lds = ((size_t) S * g.wslots + CONV_EXTRA_SLOTS) * 16;
+#define CONV_LAUNCH(SV) \
+  hipLaunchKernelGGL((conv_mfma_kernel<KT, NB, IN, SV>), grid, dim3(64 * SV), lds, s, g)
+  if (S == 4) CONV_LAUNCH(4);
+  else CONV_LAUNCH(2);
+#undef CONV_LAUNCH
 }
-
-template <int NB, int IN, int RB, int NW>
-static void launch_conv_k(int kmax, const ConvGroup &g, dim3 grid, hipStream_t s) {
-  if (kmax <= 3) launch_conv<3, NB, IN, RB, NW>(g, grid, s);
-  else if (kmax == 4) launch_conv<4, NB, IN, RB, NW>(g, grid, s);
-  else if (kmax <= 7) launch_conv<7, NB, IN, RB, NW>(g, grid, s);
-  else if (kmax <= 11) launch_conv<11, NB, IN, RB, NW>(g, grid, s);
-  else launch_conv<0, NB, IN, RB, NW>(g, grid, s);
-}
-
-template <int NB, int RB, int NW>
-static void launch_conv_in(int in_op, int kmax, const ConvGroup &g, dim3 grid, hipStream_t s) {
-  if (in_op == PTK_IN_LEAKY) launch_conv_k<NB, PTK_IN_LEAKY, RB, NW>(kmax, g, grid, s);
-  else launch_conv_k<NB, PTK_IN_PLAIN, RB, NW>(kmax, g, grid, s);
+template <int KT, int NB>
+static void launch_conv_in(int in_op, int S, const ConvGroup &g, dim3 grid, hipStream_t s) {
+  if (in_op == PTK_IN_SPLIT) return launch_conv_s<KT, NB, PTK_IN_SPLIT>(S, g, grid, s);
+  if (in_op == PTK_IN_LEAKY) launch_conv_s<KT, NB, PTK_IN_LEAKY>(S, g, grid, s);
+  else launch_conv_s<KT, NB, PTK_IN_PLAIN>(S, g, grid, s);
 }
 
 extern "C" int ptk_conv_launch(const ptk_conv_desc *dd, int ngroup, void *stream) {
@@ -1386,13 +1432,12 @@ extern "C" int ptk_conv_launch(const ptk_conv_desc *dd, int ngroup, void *stream
         order[i] = order[j];
         order[j] = t;
       }
-  const int nb = choose_nb(&dd[order[0]]);
-  int kmax = 0, in_op = -1;
+  int in_op = -1;
   int total = 0;
   const ptk_conv_desc *live[PTK_MAX_GROUP];
   for (int i = 0; i < ngroup; i++) {
     const ptk_conv_desc *d = &dd[order[i]];
-    if (!ptk_conv_mfma_ok(d) || conv_window(d, nb) > win_max(nb)) {
+    if (!ptk_conv_mfma_ok(d)) {
       set_err("ptk_conv_launch: shape outside the MFMA kernel (M %d cin %d K %d dil %d stride %d)",
               d->M, d->cin, d->K, d->dil, d->stride);
       return -1;
@@ -1405,12 +1450,12 @@ extern "C" int ptk_conv_launch(const ptk_conv_desc *dd, int ngroup, void *stream
     }
     // a row tile's weight panel is addressed through one buffer resource (the input rows are
     // bounded the same way by ptk_conv_mfma_ok)
-    if ((unsigned long long) d->K * (unsigned long long) (d->cinp / CONV_CK) * 1024ull >= (unsigned long long) PTK_OOB) {
+    if ((unsigned long long) d->K * (unsigned long long) (d->cinp / CONV_CK) * CONV_TAPB >= (unsigned long long) PTK_OOB) {
       set_err("ptk_conv_launch: weight panel (K %d, cin %d) reaches the 2 GiB range of one buffer "
               "resource", d->K, d->cin);
       return -1;
     }
-    if (d->phase_il && !(d->M == 4 * d->C4 && d->ys == 4 && d->dil == -1 && d->stride == 1 &&
+    if (d->phase_il && !(d->M == 4 * d->C4 && d->C4 % 8 == 0 && d->ys == 4 && d->dil == -1 && d->stride == 1 &&
                          d->K == 4 && ngroup == 1)) {
       set_err("ptk_conv_launch: rows interleaved by phase need a single stride-4 convT in the "
               "4-tap phase form (M %d, rows per phase %d, %d taps)", d->M, d->C4, d->K);
@@ -1421,48 +1466,86 @@ extern "C" int ptk_conv_launch(const ptk_conv_desc *dd, int ngroup, void *stream
       return -1;
     }
     if (in_op < 0) in_op = d->in_op;
-    if (d->in_op != in_op || d->in_op < PTK_IN_PLAIN || d->in_op > PTK_IN_LEAKY) {
+    if (d->in_op == PTK_IN_SPLIT && (d->xsp == nullptr || d->cin % 16 != 0 || d->bsx % 4 != 0 ||
+                                     ((uintptr_t) d->xsp & 15) != 0)) {
+      set_err("ptk_conv_launch: split planes need channels in multiples of 16 and 16-byte columns");
+      return -1;
+    }
+    if (d->ysp != nullptr && (d->C4 % 8 != 0 || d->bsy % 4 != 0 || ((uintptr_t) d->ysp & 15) != 0)) {
+      set_err("ptk_conv_launch: a split output needs channels in multiples of 8 and 16-byte columns");
+      return -1;
+    }
+    if (d->in_op != in_op || d->in_op < PTK_IN_PLAIN || d->in_op > PTK_IN_SPLIT) {
       set_err("ptk_conv_launch: grouped problems need one valid input transform");
       return -1;
     }
-    if (d->K > kmax) kmax = d->K;
     g.d[g.ngroup] = *d;
     live[g.ngroup] = d;
     g.ngroup++;
   }
   if (g.ngroup == 0) return 0;
-  int rb = 32, maxcount = 0;
-  const int S = choose_tiles(live, g.ngroup, nb, &rb), NW = S == 8 ? 8 : 4, G = NW / S;
-  g.split = S;
-  g.lg_split = S == 8 ? 3 : S == 4 ? 2 : S == 2 ? 1 : 0;
+  int maxcount = 0, S, nb, nu = 0;
+  choose_tiles(live, g.ngroup, &S, &nb);
   for (int i = 0; i < g.ngroup; i++) {
     const ptk_conv_desc *d = live[i];
     ConvProb &pi = g.info[i];
-    const long long cols = 32LL * nb * G;   // columns of one tile
-    pi.mt = (d->M + rb - 1) / rb;
-    pi.nt = (int) ((d->nq + cols - 1) / cols);
-    pi.nitem = d->batch;
-    long long n;
+    const long long cols = 32LL * nb;   // columns of one tile
+    const bool straight = d->stride == 1 && d->cin == d->cinp &&
+                          (d->K == 4 ? g.ngroup == 1 : d->K == 3 || d->K == 7 || d->K == 11);
+    const int need = straight && conv_window(d, nb) <= 32 * (nb + 1) ? nb + 1 : CONV_NU_MAX;
+    if (need > nu) nu = need;
+    pi.mt = (d->M + 31) / 32;
+    const long long nt = (d->nq + cols - 1) / cols;
+    long long nt0 = (d->nq + d->ext_l + cols - 1) / cols, n;
     if (d->batch == 1) {
-      pi.nt0 = pi.ntl = (int) ((d->nq + d->ext_l + d->ext_r + cols - 1) / cols);
-      n = (long long) pi.mt * pi.nt0;
+      nt0 = (d->nq + d->ext_l + d->ext_r + cols - 1) / cols;
+      n = pi.mt * nt0;
     } else {
-      pi.nt0 = (int) ((d->nq + d->ext_l + cols - 1) / cols);
-      pi.ntl = (int) ((d->nq + d->ext_r + cols - 1) / cols);
-      n = (long long) pi.mt * (pi.nt0 + (long long) (d->batch - 2) * pi.nt + pi.ntl);
+      n = pi.mt * (nt0 + (d->batch - 2) * nt + (d->nq + d->ext_r + cols - 1) / cols);
     }
     if (n >= (1LL << 24) || total + n >= (1LL << 31)) {
       set_err("ptk_conv_launch: %lld workgroups for one problem (the tile decode takes < 2^24)", n);
       return -1;
     }
+    // 32-bit columns: with fewer than 2^24 workgroups a column index times the stride stays below
+    // 2^31 for every window the kernel takes unless the range itself starts far out
+    const int kd = (d->K - 1) * d->dil;
+    if ((d->q0 + d->nq + d->ext_r + 64) * d->stride + (kd < 0 ? -kd : kd) >= (1LL << 31) ||
+        (d->q0 - d->ext_l) * d->stride + (kd < 0 ? kd : 0) - d->shift < -(1LL << 31) || d->lim >= (1LL << 31)) {
+      set_err("ptk_conv_launch: columns past 2^31 (q0 %lld, nq %lld, stride %d)", (long long) d->q0,
+              (long long) d->nq, d->stride);
+      return -1;
+    }
     total += (int) n;
     pi.count = (int) n;
     if (pi.count > maxcount) maxcount = pi.count;
-    pi.div_tiles = fast_div((unsigned) (pi.mt * pi.nt));
+    pi.mtnt = (int) (pi.mt * nt);
+    pi.mtnt0 = (int) (pi.mt * nt0);
+    pi.last = d->batch - 1;
+    pi.div_tiles = fast_div((unsigned) pi.mtnt);
     pi.div_mt = fast_div((unsigned) pi.mt);
     const bool il = d->phase_il != 0;
-    const bool one_phase = !il && (d->C4 == d->M || d->C4 % rb == 0);
-    pi.div_phase = fast_div(d->C4 == d->M ? 1u : (unsigned) (d->C4 / rb > 0 ? d->C4 / rb : 1));
+    const bool one_phase = !il && (d->C4 == d->M || d->C4 % 32 == 0);
+    if (one_phase && d->C4 != d->M) pi.div_phase = fast_div((unsigned) (d->C4 / 32));   // else m = 0: 0
+    pi.q0 = (int) d->q0;
+    pi.x = d->in_op == PTK_IN_SPLIT ? d->xsp : (const void *) d->x;
+    pi.w = d->w;
+    pi.scale = d->w + 2ll * (pi.mt * 32) * d->K * d->cinp;
+    pi.bias = d->bias;
+    pi.nbias4 = d->bias ? (int) (4 * (d->nbias < d->M ? d->nbias : d->M)) : 0;
+    pi.C4 = d->C4;
+    pi.K = d->K;
+    pi.dil = d->dil;
+    pi.st = d->stride;
+    pi.cin = d->cin;
+    pi.nchunk = d->cinp / CONV_CK;
+    pi.ldx4 = (int) (d->ldx * 4);
+    pi.lim = (int) d->lim;
+    pi.shift = d->shift;
+    pi.bsx = d->bsx;
+    pi.kd = kd;
+    pi.xw = conv_window(d, nb);
+    pi.in_a = d->in_a;
     pi.addt = -1;
     int naddt = 0;
     for (int e = 0; e < d->nepi; e++)
@@ -1472,27 +1555,27 @@ extern "C" int ptk_conv_launch(const ptk_conv_desc *dd, int ngroup, void *stream
     const long long lim31 = 1LL << 31, lim30 = 1LL << 30;
     bool fast = (one_phase || il) && d->ldy < (1LL << 23) && d->Lout < lim30 &&
                 (d->q0 + d->nq + d->ext_r) * d->ys + d->C4 < lim30 && d->q0 - d->ext_l >= 0 &&
-                ((long long) rb * d->ldy + d->Lout) * 4 < lim31;
+                (32 * d->ldy + d->Lout) * 4 < lim31;
     // the fast epilogue reads one tensor operand (loaded ahead of the reduction); a chain with two
     // takes the general path
     if (naddt > 1) fast = false;
     // the interleaved-phase stores have no tensor-add operand loads: such a chain takes the
-    // general path, and so do outputs where a sample pair is not 8-byte aligned (64-bit stores)
-    if (il && (pi.addt >= 0 || ((d->ldy | d->bsy) & 1) != 0 || ((uintptr_t) d->y & 7) != 0 ||
-               ((uintptr_t) d->y2 & 7) != 0))
-      fast = false;
+    // general path
+    if (il && pi.addt >= 0) fast = false;
     // PTK_CONV_FAST=0: every block through the general per-element epilogue (tests compare the
     // two epilogues)
     if (!knob(KN_CONV_FAST)) fast = false;
     if (pi.addt >= 0) {
       const long long ldt = d->epi[pi.addt].ldt;
-      fast = fast && ldt >= 0 && ldt < (1LL << 23) && ((long long) rb * ldt + d->Lout) * 4 < lim31;
+      fast = fast && ldt >= 0 && ldt < (1LL << 23) && (32 * ldt + d->Lout) * 4 < lim31;
     }
-    pi.flags = (one_phase ? PROB_ONE_PHASE : 0) | (fast ? PROB_FAST : 0) | (il ? PROB_PHASE_IL : 0);
+    pi.flags = (one_phase ? PROB_ONE_PHASE : 0) | (fast ? PROB_FAST : 0) | (il ? PROB_PHASE_IL : 0) |
+               (d->reflect_l1 ? PROB_REFLECT : 0);
     pi.ext_l = (int) d->ext_l;
     ConvEpi &ep = g.ep[i];
     ep.y = d->y;
     ep.y2 = d->y2;
+    ep.ysp = d->ysp;
     ep.bsy = d->bsy;
     ep.t = pi.addt >= 0 ? d->epi[pi.addt].t : nullptr;
     ep.bst = pi.addt >= 0 ? d->epi[pi.addt].bst : 0;
@@ -1517,11 +1600,14 @@ extern "C" int ptk_conv_launch(const ptk_conv_desc *dd, int ngroup, void *stream
   if (total == 0) return 0;
   hipStream_t s = (hipStream_t) stream;
   const dim3 grid((unsigned) maxcount, (unsigned) g.ngroup);
-  if (nb == 2) launch_conv_in<2, 32, 4>(in_op, kmax, g, grid, s);
-  else if (NW == 8 && rb == 16) launch_conv_in<1, 16, 8>(in_op, kmax, g, grid, s);
-  else if (NW == 8) launch_conv_in<1, 32, 8>(in_op, kmax, g, grid, s);
-  else if (rb == 16) launch_conv_in<1, 16, 4>(in_op, kmax, g, grid, s);
-  else launch_conv_in<1, 32, 4>(in_op, kmax, g, grid, s);
+  g.wslots = conv_slots(nu, nb);
+  for (int i = 0; i < g.ngroup; i++) g.info[i].wslots = g.wslots;
+  g.wcols = 32 * nu;
+  const bool k4 = g.ngroup == 1 && g.d[0].K == 4;
+  if (nb == 2 && k4) launch_conv_in<4, 2>(in_op, S, g, grid, s);
+  else if (nb == 2) launch_conv_in<11, 2>(in_op, S, g, grid, s);
+  else if (k4) launch_conv_in<4, 1>(in_op, S, g, grid, s);
+  else launch_conv_in<11, 1>(in_op, S, g, grid, s);
   HCHK(hipGetLastError());
   return 0;
 }
@@ -1937,6 +2023,50 @@ __global__ void avg3_leaky_kernel(const float *__restrict__ a, const float *__re
     y[i] = v >= 0.0f ? v : alpha * v;
   }
 }
+static bool al16(const void *p) { return ((uintptr_t) p & 15) == 0; }
+// leaky(((a + b) + c) / 3) of [items][C][T] tensors, as fp32 and as split planes: a thread per column
+// of eight channels.  Memory-bound (five tensors' worth of traffic).
+__global__ void __launch_bounds__(128) avg3_leaky_split_kernel(
+    const float *__restrict__ a, const float *__restrict__ b, const float *__restrict__ c,
+    float *__restrict__ y, u32x4 *__restrict__ ysp, long long ngroup, int T, float alpha) {
+  const int t = blockIdx.x * 128 + threadIdx.x;
+  if (t >= T) return;
+  for (long long g = blockIdx.y; g < ngroup; g += gridDim.y) {   // eight-channel groups of all items
+    const long long i0 = g * 8 * T + t;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const long long i = i0 + (long long) e * T;
+      const float s = ((a[i] + b[i]) + c[i]) / 3.0f;
+      v[e] = s >= 0.0f ? s : alpha * s;
+    }
+    u32x4 h, l;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      unsigned hh, ll;
+      split_pair(v[2 * e] * (float) (1 << CONV_XS), v[2 * e + 1] * (float) (1 << CONV_XS), hh, ll);
+      h[e] = hh;
+      l[e] = ll;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[i0 + (long long) e * T] = v[e];
+    ysp[g * 2 * T + t] = h;
+    ysp[(g * 2 + 1) * T + t] = l;
+  }
+}
+extern "C" int ptk_avg3_leaky_split(const float *a, const float *b, const float *c, float *y, void *ysp,
+                                    int64_t rows, int64_t T, float alpha, void *s) {
+  if (rows <= 0 || T <= 0) return 0;
+  if (rows % 8 != 0 || T >= INT_MAX - 128 || !al16(ysp)) {
+    set_err("ptk_avg3_leaky_split: %lld rows of %lld columns", (long long) rows, (long long) T);
+    return -1;
+  }
+  hipLaunchKernelGGL(avg3_leaky_split_kernel, dim3((unsigned) ((T + 127) / 128), (unsigned) (rows / 8 < 65535 ? rows / 8 : 65535)),
+                     dim3(128), 0, (hipStream_t) s, a, b, c, y, reinterpret_cast<u32x4 *>(ysp),
+                     (long long) (rows / 8), (int) T, alpha);
+  HCHK(hipGetLastError());
+  return 0;
+}
 static unsigned ew_blocks(long long n) {
   long long b = (n + 255) / 256;
   if (b > 8192) b = 8192;
@@ -1991,7 +2121,6 @@ __global__ void leaky4_kernel(const float *__restrict__ a, float *__restrict__ y
   }
   if (i0 < (n & 3)) y[(n4 << 2) + i0] = leaky1(a[(n4 << 2) + i0], alpha);
 }
-static bool al16(const void *p) { return ((uintptr_t) p & 15) == 0; }
 extern "C" int ptk_add(const float *a, const float *b, float *y, int64_t n, int epi, float alpha,
                        void *s) {
   if (n <= 0) return 0;
