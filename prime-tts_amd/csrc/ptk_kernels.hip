@@ -386,7 +386,9 @@ extern "C" int ptk_graph_destroy(void *exec) {
 #define CONV_WPE1 3
 #define CONV_PD1 4
 #define CONV_WPE2 3
-#define CONV_PD2 4
+#define CONV_PD2 3
+#define CONV_LA1 2
+#define CONV_LA2 2
 #endif
 #define CONV_XS 6          // the inputs' scale, 2^CONV_XS
 
@@ -765,27 +767,8 @@ conv_mfma_kernel(const ConvGroup g) {
   // launcher refuses it elsewhere)
   const bool phase_il = KT == 4 && (pi.flags & PROB_PHASE_IL) != 0;
   const int r_tile = fdiv(mb, pi.div_phase);
-  // Every lane loads the bias and the scale of row lane & 31 of the block, once the first chunk's
-  // loads are in flight, and the epilogue fetches each value's from the lane of its row
-  // (ds_bpermute): the loads' latency is spent behind the main loop, and no wave depends on
-  // another's write.  A row without a bias is past the buffer and reads 0.
-  float bias_r = 0.0f, scale_r = 1.0f;
-  auto load_bias = [&]() {
-    const int l = lane & 31;
-    int co = mb * 32 - r_tile * pi.C4 + l;   // conv: r_tile = 0
-    if (phase_il) co = mb * 8 + (l & 7);
-    else if (!one_phase) co = (mb * 32 + l) % pi.C4;
-    bias_r = buf_load(__builtin_amdgcn_make_buffer_rsrc((void *) pi.bias, (short) 0, pi.nbias4, PTK_BUF_WORD3),
-                      (unsigned) co * 4u, 0);
-    scale_r = pi.scale[mb * 32 + l];
-  };
-  // bias and scale of row `row` of the block (every lane of the wave must be active)
-  auto bias_of = [&](int row) {
-    return __int_as_float(__builtin_amdgcn_ds_bpermute(row * 4, __float_as_int(bias_r)));
-  };
-  auto scale_of = [&](int row) {
-    return __int_as_float(__builtin_amdgcn_ds_bpermute(row * 4, __float_as_int(scale_r)));
-  };
+  // Every lane loads the scale of row lane & 31 of the block: NaN where a row has no fp16 form.
+  float scale_r = 0.0f;
   const int half = lane >> 5;     // which eight of a chunk's channels this lane feeds
   const int l32 = lane & 31;
   const int dmin = min(pi.kd, 0);
@@ -857,7 +840,7 @@ conv_mfma_kernel(const ConvGroup g) {
     constexpr int KC = decltype(kc)::value, NU = decltype(nuc)::value;
     constexpr bool MASK = decltype(mask)::value;
     constexpr int PS = NU * 32;   // plane stride (16-byte slots)
-    constexpr int PD = KC == 0 ? 1 : NB == 1 ? CONV_PD1 : CONV_PD2;   // slices the A operands are loaded ahead of their use
+    constexpr int PDM = NB == 1 ? CONV_PD1 : CONV_PD2, PD = KC == 0 ? 1 : KC < PDM ? KC : PDM;   // slices A is loaded ahead
     constexpr bool SPLIT = IN == PTK_IN_SPLIT;
     float raw[NU][8], mag[NU];      // fp32 input: what is loaded, its largest magnitude
     u32x4 raws[NU][2];              // split planes: what is loaded
@@ -935,7 +918,7 @@ conv_mfma_kernel(const ConvGroup g) {
     for (int u = 0; u < NU; u++) load_unit(rx, u, 0);
 #pragma unroll
     for (int k = 0; k < PD; k++) ahead[k] = wa(rw, min(k, last));
-    load_bias();
+    scale_r = pi.scale[mb * 32 + l32];
     {
       const __amdgpu_buffer_rsrc_t rx1 = x_rsrc(nch > 1);
 #pragma unroll
@@ -956,12 +939,14 @@ conv_mfma_kernel(const ConvGroup g) {
         Parts a[KC + PD];
 #pragma unroll
         for (int k = 0; k < PD; k++) a[k] = ahead[k];
-        Parts q = col(0, 0);
+        constexpr int LA = NB == 1 ? CONV_LA1 : CONV_LA2;   // steps the B operands are read ahead
+        Parts q[NS + LA];
+#pragma unroll
+        for (int s = 0; s < LA; s++) q[s] = col(s / NB, s % NB);
 #pragma unroll
         for (int s = 0; s < NS; s++) {
           const int k = s / NB, nb = s % NB;
-          Parts qn = q;
-          if (s + 1 < NS) qn = col((s + 1) / NB, (s + 1) % NB);
+          if (s + LA < NS) q[s + LA] = col((s + LA) / NB, (s + LA) % NB);
           if (nb == 0) a[k + PD] = wa(rw, k + PD < KC ? j * KC + k + PD : min(j * KC + k + PD, last));
           // the next chunk's split over the last two thirds of the steps
 #pragma unroll
@@ -970,9 +955,8 @@ conv_mfma_kernel(const ConvGroup g) {
               split_unit(i / 4, i % 4);
               if (i % 4 == 3) load_unit(rx2, i / 4, j + 2);
             }
-          mfma3(a[k], q, nb);
+          mfma3(a[k], q[s], nb);
           __builtin_amdgcn_sched_barrier(0);
-          q = qn;
         }
 #pragma unroll
         for (int k = 0; k < PD; k++) ahead[k] = a[KC + k];
@@ -1061,7 +1045,7 @@ conv_mfma_kernel(const ConvGroup g) {
   const bool narrow = XW <= 32 * (NB + 1);
   // channel padding in the last chunk, a stride or another K: the rolled body
   const int straight = cin == nchunk * CONV_CK && st == 1 ? K : 0;
-  if (nch == 0) load_bias();
+  if (nch == 0) scale_r = pi.scale[mb * 32 + l32];
   else if (KT == 4 && straight == 4 && narrow) run(std::integral_constant<int, KT == 4 ? 4 : 0>{}, nomask, few);
   else if (KT == 11 && straight == 11 && narrow) run(std::integral_constant<int, KT == 11 ? 11 : 0>{}, nomask, few);
   else if (KT == 11 && straight == 11) run(std::integral_constant<int, KT == 11 ? 11 : 0>{}, nomask, all);
@@ -1072,23 +1056,22 @@ conv_mfma_kernel(const ConvGroup g) {
   // Epilogue: the S partial sums of a block are added in wave order through LDS, then bias, the
   // epilogue chain and one store per output.  Lane (l32, half) holds, for column block nb, the 16
   // values v of column q0 + 32*nb + l32 at rows 8*(v >> 2) + 4*half + (v & 3) of the block.  Wave w
-  // finishes the NMAX = 16 / S values from v0 = w * NMAX, in groups of GRP <= 4 (rows of one v >> 2).
-  constexpr int NMAX = 16 / S, GRP = NMAX < 4 ? NMAX : 4, NG = NMAX / GRP;
+  // finishes the NMAX = 16 / S values from v0 = w * NMAX, in groups of GRP = 4 (rows of one v >> 2).
+  constexpr int NMAX = 16 / S, GRP = 4, NG = NMAX / GRP;
   const int v0 = w * NMAX;
   const int addt = pi.addt;   // the chain's residual add, if any
   auto vrow = [&](int i) { return 8 * ((v0 + i) >> 2) + 4 * half + ((v0 + i) & 3); };   // of value i
   unsigned mine = ~0u;   // bit nb: this pass stores the lane's column of block nb
   bool again = false;    // some column is left to the second pass
-  for (int pass = 0;; pass++) {
-  // (an opaque copy of the problem index: the compiler would otherwise load everything the rare
-  // paths read ahead of the loop)
-  int pe = p;
-  asm volatile("" : "+s"(pe));
-  const ptk_conv_desc &d = g.d[pe];
+  // (once for each pass, not a loop over them: the compiler would compute everything the rare paths
+  // need ahead of the loop, some 200 instructions)
+  auto finish = [&](auto passc) {
+  constexpr int pass = decltype(passc)::value;
+  const ptk_conv_desc &d = g.d[p];
   // Each wave writes its partial sums over its own staging area, which only it reads, so no wave
   // waits for the others before writing: [nb][v >> 2][lane] float4.
   int *const flags = reinterpret_cast<int *>(smem + S * wslots);
-  if constexpr (S > 1) {
+  {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     f32x4 *red = reinterpret_cast<f32x4 *>(xs);
 #pragma unroll
@@ -1102,17 +1085,15 @@ conv_mfma_kernel(const ConvGroup g) {
       }
   }
   const bool alarm = pass == 0 && __ballot(odd || scale_r != scale_r) != 0;
-  if (S > 1 && pass == 0 && lane == 0) flags[w] = alarm;
+  if (pass == 0 && lane == 0) flags[w] = alarm;
   // the barrier behind the partial sums; then, in a workgroup that was alarmed, the columns that
   // are left to the second pass
   auto reduce_wait = [&]() {
-    if constexpr (S > 1) __syncthreads();
+    __syncthreads();
     if (pass != 0) return;
-    int any = alarm;
-    if constexpr (S > 1) {
+    int any = flags[0];
 #pragma unroll
-      for (int i = 0; i < S; i++) any |= flags[i];
-    }
+    for (int i = 1; i < S; i++) any |= flags[i];
     if (__builtin_expect(__builtin_amdgcn_readfirstlane(any) == 0, 1)) return;
     float *const cm = reinterpret_cast<float *>(smem + S * wslots + 2);   // per window column
     for (int i = threadIdx.x; i < XW; i += 64 * S) {
@@ -1135,25 +1116,17 @@ conv_mfma_kernel(const ConvGroup g) {
     }
     again = __ballot(mine != (1u << NB) - 1) != 0;
   };
-  // The S partial sums of GRP values in wave order.
-  auto reduced = [&](int nb, int gg, float *val) {
-    if constexpr (S > 1) {
-      const int v = v0 + gg * GRP;
-      typedef float vec __attribute__((ext_vector_type(GRP)));
-      vec part[S];
+  // The S partial sums of a group's values, in wave order.
+  auto reduced = [&](int nb, int gg) {
+    const int v = v0 + gg * GRP;
+    f32x4 part[S];
 #pragma unroll
-      for (int i = 0; i < S; i++)
-        part[i] = *reinterpret_cast<const vec *>(reinterpret_cast<const float *>(smem + i * wslots) +
-                                                 (((nb * 4 + (v >> 2)) * 64 + lane) * 4 + (v & 3)));
-      vec sum = part[0];
+    for (int i = 0; i < S; i++)
+      part[i] = reinterpret_cast<const f32x4 *>(smem + i * wslots)[(nb * 4 + (v >> 2)) * 64 + lane];
+    f32x4 sum = part[0];
 #pragma unroll
-      for (int i = 1; i < S; i++) sum += part[i];
-#pragma unroll
-      for (int i = 0; i < GRP; i++) val[gg * GRP + i] = sum[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < GRP; i++) val[gg * GRP + i] = acc[nb][gg * GRP + i];
-    }
+    for (int i = 1; i < S; i++) sum += part[i];
+    return sum;
   };
   // Fast path: a full block whose rows are consecutive output channels (conv, or a convT block
   // inside one phase), with every index of the output, its LeakyReLU copy and the residual inside
@@ -1164,7 +1137,7 @@ conv_mfma_kernel(const ConvGroup g) {
   // op by op over a lane's values, one branch per op.  A convT block with its rows interleaved by
   // phase (phase_il) holds 8 whole channels.
   if ((pi.flags & PROB_FAST) && (one_phase || phase_il) && mb * 32 + 32 <= pi.M) {
-    const ConvEpi ep = g.ep[pe];
+    const ConvEpi ep = g.ep[p];
     // first channel of the block
     const long long row0 = phase_il ? (long long) mb * 8 : (long long) mb * 32 - (long long) r_tile * ep.C4;
     const int ldy32 = ep.ldy, ldt32 = ep.ldt;
@@ -1195,6 +1168,20 @@ conv_mfma_kernel(const ConvGroup g) {
           rv[nb][i] = buf_load(rt, (unsigned) (4 * half * ldt32 + cl) * 4u, (unsigned) (urow(i) * ldt32) * 4u);
       }
     }
+    // the bias and scale of a lane's rows (a row without a bias is past the buffer and reads 0), in
+    // flight with the residual while the partial sums are written
+    f32x4 bias[NG], scale[NG];
+    {
+      const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *) pi.bias, (short) 0, pi.nbias4, PTK_BUF_WORD3);
+#pragma unroll
+      for (int gg = 0; gg < NG; gg++) {
+        const int rg = urow(gg * GRP);
+        bias[gg] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+            rb, (unsigned) ((int) row0 + 4 * half + (phase_il ? 0 : rg)) * 4u, 0, 0));
+        if constexpr (pass == 0) scale[gg] = *reinterpret_cast<const f32x4 *>(pi.scale + mb * 32 + 4 * half + rg);
+        else scale[gg] = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
+      }
+    }
     reduce_wait();
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
@@ -1203,10 +1190,11 @@ conv_mfma_kernel(const ConvGroup g) {
       const bool oq = q < qend32 && (mine >> nb & 1);
       float val[NMAX];
 #pragma unroll
-      for (int gg = 0; gg < NG; gg++) reduced(nb, gg, val);
+      for (int gg = 0; gg < NG; gg++) {
+        const f32x4 sum = reduced(nb, gg);
 #pragma unroll
-      for (int i = 0; i < NMAX; i++)
-        val[i] = __fadd_rn(bias_of(4 * half + urow(i)), val[i] * scale_of(4 * half + urow(i)));
+        for (int i = 0; i < GRP; i++) val[gg * GRP + i] = fmaf(sum[i], scale[gg][i], bias[gg][i]);
+      }
       // The chain.  The decoder's two chains, a LeakyReLU and a tensor add (the chain's one, the
       // launcher's rule), have their own code; any other goes op by op.
       if (ep.ops == PTK_EPI_ADDT) {
@@ -1257,14 +1245,9 @@ conv_mfma_kernel(const ConvGroup g) {
           }
           const unsigned vs = (unsigned) cg * 16u + (unsigned) half * 8u;
           const unsigned ss = (unsigned) ((rg >> 3) * 8 * ldy32) * 4u + (unsigned) (rg & 3) * 2u;
-          if constexpr (GRP == 4) {
-            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-            __builtin_amdgcn_raw_buffer_store_b64(u32x2{h[0], h[1]}, rys, vs, ss, 0);
-            __builtin_amdgcn_raw_buffer_store_b64(u32x2{l[0], l[1]}, rys, vs, ss + 16u * (unsigned) ldy32, 0);
-          } else {
-            __builtin_amdgcn_raw_buffer_store_b32(h[0], rys, vs, ss, 0);
-            __builtin_amdgcn_raw_buffer_store_b32(l[0], rys, vs, ss + 16u * (unsigned) ldy32, 0);
-          }
+          typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+          __builtin_amdgcn_raw_buffer_store_b64(u32x2{h[0], h[1]}, rys, vs, ss, 0);
+          __builtin_amdgcn_raw_buffer_store_b64(u32x2{l[0], l[1]}, rys, vs, ss + 16u * (unsigned) ldy32, 0);
         }
       }
     }
@@ -1280,16 +1263,15 @@ conv_mfma_kernel(const ConvGroup g) {
   const bool phase_rows = C4 != M;
   const long long qend = d.q0 + d.nq + (last_item ? d.ext_r : 0);
   reduce_wait();
-#pragma unroll
+#pragma unroll 1
   for (int nb = 0; nb < NB; nb++) {
     const long long q = (long long) q0 + 32 * nb + l32;
-    float val[NMAX];
+#pragma unroll 1
+    for (int gg = 0; gg < NG; gg++) {
+    const f32x4 sum = reduced(nb, gg);
 #pragma unroll
-    for (int gg = 0; gg < NG; gg++) reduced(nb, gg, val);
-#pragma unroll
-    for (int i = 0; i < NMAX; i++) {
-      const int m = mb * 32 + vrow(i);
-      float v = __fadd_rn(bias_of(vrow(i)), val[i] * scale_of(vrow(i)));   // all lanes active here
+    for (int i = 0; i < GRP; i++) {
+      const int m = mb * 32 + vrow(gg * GRP + i);
       if (m >= M || q >= qend || !(mine >> nb & 1)) continue;
       int co = m, r = 0;
       if (phase_il) {
@@ -1301,6 +1283,7 @@ conv_mfma_kernel(const ConvGroup g) {
       }
       const long long col = q * ys + r - ypad;
       if (col < 0 || col >= Lout) continue;
+      float v = fmaf(sum[i], pass == 0 ? pi.scale[m] : 1.0f, d.bias != nullptr && co < d.nbias ? d.bias[co] : 0.0f);
       for (int e = 0; e < nepi; e++) v = epi_apply(v, d.epi[e], b, co, col);
       const long long yi = (long long) co * ldy + col;
       yb[yi] = v;
@@ -1314,20 +1297,21 @@ conv_mfma_kernel(const ConvGroup g) {
         ys16[8 * ldy] = (unsigned short) l;
       }
     }
+    }
   }
   }
-  if (__builtin_expect(!again, 1)) break;
+  };
+  finish(std::integral_constant<int, 0>{});
+  if (__builtin_expect(!again, 1)) return;
   // the columns left over, from fp32 operands
-  again = false;
   mine = ~mine;
-  scale_r = 1.0f;
 #pragma unroll
   for (int nb = 0; nb < NB; nb++)
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[nb][v] = 0.0f;
   __syncthreads();   // every wave is done with the first pass's partial sums
-  if (nch > 0) run32(d);
-  }
+  if (nch > 0) run32(g.d[p]);
+  finish(std::integral_constant<int, 1>{});
 }
 
 static int conv_window(const ptk_conv_desc *d, int nb) {
@@ -1388,6 +1372,28 @@ static void choose_tiles(const ptk_conv_desc *const *ds, int n, int *S_out, int 
   }
   *nb_out = nb2_ok && (env_nb == 2 || (env_nb != 1 && wgs >= 200)) ? 2 : 1;
   *S_out = env_s == 2 || env_s == 4 ? env_s : item >= 640 ? 2 : 4;
+}
+
+// Order of three grouped problems (given heaviest first).  Workgroups are handed round the CUs in
+// order, so in a launch that is resident at once the last problem's land on the CUs the first one's
+// went to.  Heaviest first is right once CUs take several rounds; below that the heaviest belongs
+// second, so that the lightest joins the middle one (per depth at C 256, T 904: 33.1 -> 31.3 us,
+// T 720: 31.8 -> 28.5), and with two-wave workgroups, a problem of up to one per CU, last but the
+// lightest second (C 128, T 3616: 35.1 -> 33.1 us, T 3472: 35.1 -> 32.6).
+static void order_problems(const ptk_conv_desc **ds, int n, int S, int nb) {
+  if (n != 3) return;
+  long long total = 0, most = 0;
+  for (int i = 0; i < 3; i++) {
+    const long long wgs = (long long) ds[i]->batch * ((ds[i]->M + 31) / 32) * ((ds[i]->nq + 32 * nb - 1) / (32 * nb));
+    total += wgs;
+    if (wgs > most) most = wgs;
+  }
+  const int cus = 256;
+  if (total > 12 / S * cus) return;   // more than are resident at once (three waves per SIMD)
+  const int a = S == 2 && most <= cus ? 1 : 0;   // swap the last two, or the first two
+  const ptk_conv_desc *t = ds[a];
+  ds[a] = ds[a + 1];
+  ds[a + 1] = t;
 }
 
 extern "C" int ptk_conv_mfma_ok(const ptk_conv_desc *d) {
@@ -1479,15 +1485,16 @@ extern "C" int ptk_conv_launch(const ptk_conv_desc *dd, int ngroup, void *stream
       set_err("ptk_conv_launch: grouped problems need one valid input transform");
       return -1;
     }
-    g.d[g.ngroup] = *d;
     live[g.ngroup] = d;
     g.ngroup++;
   }
   if (g.ngroup == 0) return 0;
   int maxcount = 0, S, nb, nu = 0;
   choose_tiles(live, g.ngroup, &S, &nb);
+  order_problems(live, g.ngroup, S, nb);
   for (int i = 0; i < g.ngroup; i++) {
     const ptk_conv_desc *d = live[i];
+    g.d[i] = *d;
     ConvProb &pi = g.info[i];
     const long long cols = 32LL * nb;   // columns of one tile
     const bool straight = d->stride == 1 && d->cin == d->cinp &&
