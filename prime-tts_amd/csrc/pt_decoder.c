@@ -5,11 +5,11 @@
  *   ups.0 convT 512->256 K16 s4 p6                  one phase-form GEMM (4 phases = 1024 rows)
  *   MRF-256: per depth j, one grouped launch of the three branches' c1 (input already
  *            LeakyReLU'd by its producer, epilogue leaky), then one of their c2 (epilogue adds the
- *            residual and, for depths 0 and 1, also writes the LeakyReLU'd copy the next depth's
- *            c1 reads)  -> 6 launches, three branch outputs left in HBM.  ups.0 / ups.1 write
- *            their output and its LeakyReLU'd copy the same way.
+ *            residual and, for depths 0 and 1, also writes its LeakyReLU as the split planes the
+ *            next depth's c1 reads)  -> 6 launches, three branch outputs left in HBM.  conv_pre,
+ *            ups.0 and ups.1 write their split planes the same way.
  *   ups.1 convT 256->128 over leaky(((b0 + b1) + b2) / 3, 0.1), formed once by one elementwise
- *            pass (cheaper than re-forming it in each of ups.1's 16 row blocks' staging)
+ *            pass, in fp32 and as split planes
  *   MRF-128 as above
  *   conv_post 128->72 K7 over leaky((...)/3, 0.01), formed the same way, through the (1, 0)
  *            reflection pad

@@ -1,14 +1,13 @@
 // ptk_kernels.hip -- gfx950 (MI355X) kernels of the PrimeTTS conv hot path, and the thin C-ABI
 // layer (ptk.h) through which the C host code reaches them.
 //
-// Wide Conv1d / ConvTranspose1d run as one implicit GEMM on the fp32 matrix cores
-// (v_mfma_f32_32x32x2_f32, or v_mfma_f32_16x16x4_f32 for 16-row tiles when one batch item's grid
-// is too small to fill the chip): GEMM rows are output channels (convT: phase rows r*C4 + co, the
-// reference's packed phase layout), columns are output positions, the reduction runs over
-// (tap, input channel).  im2col never exists: each wave stages a window of input columns per
-// channel chunk in LDS and reads it K times at the K tap shifts.  The four waves of a workgroup
-// (eight for the 8-way split of single problems that leave one wave per SIMD) split the input
-// channels and reduce through LDS in a fixed order (deterministic), then the
+// Wide Conv1d / ConvTranspose1d run as one implicit GEMM on the matrix cores: fp32 products as
+// three fp16 ones (v_mfma_f32_32x32x16_f16, fp32 accumulation), or on v_mfma_f32_32x32x2_f32 where
+// the operands do not fit fp16's range.  GEMM rows are output channels (convT: phase rows
+// r*C4 + co, the reference's packed phase layout), columns are output positions, the reduction
+// runs over (tap, input channel).  im2col never exists: each wave stages a window of input columns
+// per channel chunk in LDS and reads it K times at the K tap shifts.  The two or four waves of a
+// workgroup split the input channels and reduce through LDS in a fixed order (deterministic), then the
 // epilogue (bias, LeakyReLU/ReLU/scalar ops, residual / branch-sum tensor adds, division) is
 // applied on the accumulator values right before the single store.
 #include <hip/hip_runtime.h>
@@ -723,6 +722,12 @@ __device__ __forceinline__ bool conv_alarm_free(float m) {
 // pass watches the magnitudes it stages (a unit's own channels, so it may raise a false alarm but
 // misses nothing); only a workgroup it alarms looks at its columns one by one.
 //
+// Bound by the matrix cores on large launches (552 TFLOP/s of fp32 products at the rate the card
+// sustains, 150 on the fp32 matrix cores), by the way in and out of a workgroup on small ones.
+// Against the fp32-MFMA kernel it replaced: MRF-256 stack at T 904 149 -> 82 us, MRF-128 at T 3616
+// 154 -> 98 us, conv_pre at T 226 6.35 -> 5.6 us, ups.0 11.4 -> 9.5 us, a T 226 decode 345 -> 221 us
+// and eight in a batch 2141 -> 987 us; errors against 64 bits 0.6-0.8 of what they were.
+//
 // KT: the taps the straight-line bodies are built for (11: K = 11, 7 and 3; 4: K = 4, the convT
 // phase form); any other K goes through a rolled loop.  IN: input transform (PTK_IN_*).
 template <int KT, int NB, int IN, int S>
@@ -1356,6 +1361,9 @@ extern "C" void ptk_knobs_reload(void) {
 
 // Tile shape: the channel split S in {2, 4} (PTK_CONV_SPLIT overrides) and the column blocks per
 // wave NB in {1, 2} (PTK_CONV_NB).
+// Measured: S = 2 against 4 at C 128, T 3616, batch 8 159-165 against 175-195 us, at C 256, T 904 37
+// against 30 us; NB = 2 against 1 for the MRF-256 group at T 904 30 against 33 us, at T 252 22.8
+// against 17.8 us, ups.0 at T 226 12.5 against 10.3 us, conv_pre at batch 8 13 against 16.6 us.
 // S fixes the order in which a block's partial sums are added, so it is chosen from one batch item's
 // grid (of nq_shape columns when the launch covers a sub-range): a batched item's result is
 // bit-identical to the same item alone.  NB changes no bit and is chosen from the whole launch.
@@ -2033,6 +2041,8 @@ __global__ void avg3_leaky_kernel(const float *__restrict__ a, const float *__re
 static bool al16(const void *p) { return ((uintptr_t) p & 15) == 0; }
 // leaky(((a + b) + c) / 3) of [items][C][T] tensors, as fp32 and as split planes: a thread per column
 // of eight channels.  Memory-bound (five tensors' worth of traffic).
+// Bound by HBM: at batch 8, T 226 9.1 us (C 256) and 11.9 us (C 128); the fp32-only pass it replaced
+// took 5.6 and 9.7 us, and the convs behind it then split their input per row block.
 __global__ void __launch_bounds__(128) avg3_leaky_split_kernel(
     const float *__restrict__ a, const float *__restrict__ b, const float *__restrict__ c,
     float *__restrict__ y, u32x4 *__restrict__ ysp, long long ngroup, int T, float alpha) {
