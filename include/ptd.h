@@ -267,6 +267,10 @@ void ptd_debug_reload_env(void);
  * arena set to `byte` on its stream (0xff makes every float NaN, so a column read before any
  * launch wrote it poisons what depends on it).  Synchronous.  0 / -1. */
 int ptd_debug_fill_arena(pt_ctx *c, int byte);
+/* Tests of which path a conv takes (no counterpart in the reference): how many workgroups of the
+ * conv kernel, since the library was loaded, looked at their columns one by one ([0]) and computed
+ * some of them again from fp32 operands ([1]).  Waits for the device.  0 / -1. */
+int ptd_debug_conv_stats(uint64_t out[2]);
 int ptd_h2d(pt_ctx *c, void *dst, const void *src, size_t bytes);   /* synchronous */
 int ptd_d2h(pt_ctx *c, void *dst, const void *src, size_t bytes);   /* synchronous */
 int ptd_sync(pt_ctx *c);                        /* wait for the context's stream */

@@ -1060,6 +1060,13 @@ int ptd_debug_fill_arena(pt_ctx *c, int byte) {
   }
   return 0;
 }
+int ptd_debug_conv_stats(uint64_t out[2]) {
+  if (ptk_init() || ptk_conv_stats(out)) {
+    PT_LOG("conv statistics: %s", ptk_last_error());
+    return -1;
+  }
+  return 0;
+}
 int ptd_h2d(pt_ctx *c, void *dst, const void *src, size_t bytes) {
   if (!c || !c->use_cuda) return -1;
   return (ptk_h2d_async(dst, src, bytes, c->g_stream) || ptk_stream_sync(c->g_stream)) ? -1 : 0;

@@ -164,6 +164,10 @@ int ptk_h2f(float *dst, const uint16_t *src, int64_t n, void *s);
 int ptk_conv_launch(const ptk_conv_desc *d, int ngroup, void *s);
 /* 1 when the MFMA kernel covers this problem's shape; else the caller uses the SIMT path */
 int ptk_conv_mfma_ok(const ptk_conv_desc *d);
+/* workgroups of the conv kernel, on the current device since the library was loaded, that looked at
+ * their columns one by one, and that computed some of them again from fp32 operands; waits for the
+ * device */
+int ptk_conv_stats(uint64_t out[2]);
 
 /* SIMT fallbacks over the PACKED layouts, for narrow shapes (cout4 < 16, tiny cin, huge K*dil):
  * conv: X rows of ldx with in-kernel padding by `shift`; convT: the phase/tap form.  The conv's

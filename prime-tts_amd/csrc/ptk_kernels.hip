@@ -618,7 +618,8 @@ struct ConvProb {
   int kd, xw;                     // (K - 1) * dil; window columns
   float in_a;
   int wslots;                     // ConvGroup's: LDS of one wave, in 16-byte slots
-  int pad[8];
+  int qend, ext_r;                // a middle item's column end; the last item's goes ext_r further
+  int pad[6];
 };
 // every row block lies inside one phase (conv, or C4 % 32 == 0)
 #define PROB_ONE_PHASE 1
@@ -710,6 +711,10 @@ __device__ __forceinline__ bool conv_alarm_free(float m) {
   return m < 1023.0f && (m >= 0.00390625f || m == 0.0f);
 }
 
+// Workgroups since the library was loaded that looked at their columns one by one / ran the second
+// pass (counted on those rare paths only).
+__device__ unsigned long long conv_stat[2];
+
 // One workgroup = S waves on one block of 32 rows x 32*NB columns.  The waves take disjoint runs of
 // the 16-channel chunks and are reduced through LDS in wave order (deterministic).  Each product of
 // two fp32 values is taken as three fp16 products on v_mfma_f32_32x32x16_f16 (hi.lo, lo.hi, hi.hi;
@@ -779,11 +784,16 @@ conv_mfma_kernel(const ConvGroup g) {
   const int dmin = min(pi.kd, 0);
   const int XW = pi.xw;
   const int cmin = q0 * st + dmin - pi.shift;   // the window's first virtual column
+  // Columns from here on are staged as zeros: past the row, past the window, or read by no output
+  // of this item.  The last tile of an item rounds up past its columns, and in a launch over part
+  // of the columns what lies there may never have been written.
+  const int cend = max(min(lim, (min(q0 + 32 * NB, pi.qend + (last_item ? pi.ext_r : 0)) - 1) * st +
+                                    max(pi.kd, 0) - pi.shift + 1), 0);
   u32x4 *const xs = smem + w * wslots;   // this wave's staging planes
 
   // Window columns this lane stages, fixed for the wave: unit u, column 32u + l32, channels 8*half
   // .. 8*half + 7 of the chunk; byte offset of the first, or an offset the buffer range check turns
-  // into 0 (columns outside [0, lim), past the window).  The row step and the chunk are wave-uniform
+  // into 0 (columns outside [0, cend)).  The row step and the chunk are wave-uniform
   // and go into the scalar offset.
   const long long xoff = b * pi.bsx;
   const unsigned nrec = (unsigned) cin * ldx4;
@@ -795,11 +805,11 @@ conv_mfma_kernel(const ConvGroup g) {
     if (pi.flags & PROB_REFLECT) {   // (column 0 reads column 1: the window holds 0 and 1 together)
 #pragma unroll
       for (int u = 0; u < CONV_NU_MAX; u++, c += 32)
-        voff[u] = (unsigned) c < (unsigned) lim && l32 + 32 * u < XW ? (unsigned) (c == 0 ? 1 : c - 1) * CB + h8 : PTK_OOB;
+        voff[u] = (unsigned) c < (unsigned) cend ? (unsigned) (c == 0 ? 1 : c - 1) * CB + h8 : PTK_OOB;
     } else {
 #pragma unroll
       for (int u = 0; u < CONV_NU_MAX; u++, c += 32)
-        voff[u] = (unsigned) c < (unsigned) lim && l32 + 32 * u < XW ? (unsigned) c * CB + h8 : PTK_OOB;
+        voff[u] = (unsigned) c < (unsigned) cend ? (unsigned) c * CB + h8 : PTK_OOB;
     }
   }
 
@@ -1100,11 +1110,12 @@ conv_mfma_kernel(const ConvGroup g) {
 #pragma unroll
     for (int i = 1; i < S; i++) any |= flags[i];
     if (__builtin_expect(__builtin_amdgcn_readfirstlane(any) == 0, 1)) return;
+    if (threadIdx.x == 0) atomicAdd(&conv_stat[0], 1ull);
     float *const cm = reinterpret_cast<float *>(smem + S * wslots + 2);   // per window column
     for (int i = threadIdx.x; i < XW; i += 64 * S) {
       const int c = cmin + i, pc = pi.flags & PROB_REFLECT ? (c == 0 ? 1 : c - 1) : c;
       float m = 0.0f;
-      if (c >= 0 && c < lim)
+      if (c >= 0 && c < cend)
         for (int ci = 0; ci < cin; ci++) m = max_mag(m, xform32(d.x[xoff + (long long) ci * d.ldx + pc]), 0.0f);
       cm[i] = m;
     }
@@ -1309,6 +1320,7 @@ conv_mfma_kernel(const ConvGroup g) {
   finish(std::integral_constant<int, 0>{});
   if (__builtin_expect(!again, 1)) return;
   // the columns left over, from fp32 operands
+  if (threadIdx.x == 0) atomicAdd(&conv_stat[1], 1ull);
   mine = ~mine;
 #pragma unroll
   for (int nb = 0; nb < NB; nb++)
@@ -1411,6 +1423,12 @@ extern "C" int ptk_conv_mfma_ok(const ptk_conv_desc *d) {
   // 32-bit buffer offsets: every row offset plus the out-of-range marker must stay below 2^32
   if ((unsigned long long) d->cinp * (unsigned long long) d->ldx * 4ULL >= 0x80000000ULL) return 0;
   return 1;
+}
+
+extern "C" int ptk_conv_stats(uint64_t out[2]) {
+  HCHK(hipDeviceSynchronize());
+  HCHK(hipMemcpyFromSymbol(out, HIP_SYMBOL(conv_stat), 2 * sizeof(uint64_t)));
+  return 0;
 }
 
 template <int KT, int NB, int IN>
@@ -1587,6 +1605,8 @@ extern "C" int ptk_conv_launch(const ptk_conv_desc *dd, int ngroup, void *stream
     pi.flags = (one_phase ? PROB_ONE_PHASE : 0) | (fast ? PROB_FAST : 0) | (il ? PROB_PHASE_IL : 0) |
                (d->reflect_l1 ? PROB_REFLECT : 0);
     pi.ext_l = (int) d->ext_l;
+    pi.qend = (int) (d->q0 + d->nq);
+    pi.ext_r = (int) d->ext_r;
     ConvEpi &ep = g.ep[i];
     ep.y = d->y;
     ep.y2 = d->y2;

@@ -518,6 +518,26 @@ def test_window_columns_change_no_sample(env, T, win, cx, knob_env):
     dz.free(); dw.free()
 
 
+@pytest.mark.parametrize("T,win,cx", [(1500, 96, 16), (400, 64, 12), (48, 48, 16)])
+def test_windowed_decode_judges_no_unread_column(env, T, win, cx):
+    """A launch over part of the columns neither stages nor judges the ones beside them, which
+    nobody wrote: with the arena full of NaN a windowed decode sends no workgroup to look at its
+    columns one by one (ordinary latents: a handful of values at most may call for it)."""
+    ctx, model, ws, bs = env
+    say(f"windowed decode's unread columns T={T} win={win} ctx={cx}")
+    z = synth.latent(T, 4300 + T)
+    dz, dw = dev_of(ctx, z), pkg.DevBuf(256 * T)
+    n0, n1 = (C.c_uint64 * 2)(), (C.c_uint64 * 2)()
+    assert ctx.lib.ptd_debug_fill_arena(ctx.ptr, 0xFF) == 0
+    assert ctx.lib.ptd_debug_conv_stats(n0) == 0
+    assert ctx.lib.ptd_decode_windows(ctx.ptr, model.ptr, dz.ptr, T, win, cx, dw.ptr) == 0
+    assert ctx.lib.ptd_debug_conv_stats(n1) == 0
+    say(f"  looked at columns: {n1[0] - n0[0]} workgroups, second pass: {n1[1] - n0[1]}")
+    # the decode's conv launches have thousands of workgroups; unread columns alarmed hundreds
+    assert n1[0] - n0[0] <= 16 and n1[1] == n0[1]
+    dz.free(); dw.free()
+
+
 @pytest.mark.parametrize("tout,grid", [("256", "7"), ("1024", "3"), ("512", "-1"), ("256", "8"),
                                        ("1024", "24")])
 def test_window_tail_tiles_and_grid_change_no_sample(env, tout, grid, knob_env):
