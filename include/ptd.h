@@ -111,7 +111,14 @@ int ptd_tail(pt_ctx *c, const ptd_model *m, const float *p, int64_t L, int batch
 
 /* Run decoder layer i (0..39) alone: conv (x [batch][cin][T] -> y [batch][cout4][Tout]) or convT
  * (x [batch][cin][T] -> y [batch][cout4][Lout]).  in_leaky > 0 applies LeakyReLU(in_leaky) to
- * the input as it is read; epi_leaky > 0 applies it to the output.  Asynchronous. */
+ * the input as it is read; epi_leaky > 0 applies it to the output.  Asynchronous.
+ *
+ * Precision of every wide conv and convT (this one, pt_v21_conv / pt_v21_convT, the decodes): products
+ * are summed in fp32.  With A = sum of |w x| over an output's products and n the nonzero weights of
+ * its row, the error is that of an fp32 sum (n 2^-24 A in the worst order) plus at most
+ * (n/2 + 8) 2^-24 A, at any input scale and for any mix of magnitudes.  Full speed needs inputs below
+ * 2^12 and outputs that are not far below what their inputs' spread would make them; others are
+ * computed a second time from the fp32 operands. */
 int ptd_layer(pt_ctx *c, const ptd_model *m, int layer, const float *x, int64_t T, int batch,
               float *y, float in_leaky, float epi_leaky);
 /* The same over a part of the GEMM columns (no counterpart in the reference): cols = {q0, nq,
@@ -268,8 +275,9 @@ void ptd_debug_reload_env(void);
  * launch wrote it poisons what depends on it).  Synchronous.  0 / -1. */
 int ptd_debug_fill_arena(pt_ctx *c, int byte);
 /* Tests of which path a conv takes (no counterpart in the reference): how many workgroups of the
- * conv kernel, since the library was loaded, looked at their columns one by one ([0]) and computed
- * some of them again from fp32 operands ([1]).  Waits for the device.  0 / -1. */
+ * conv kernel, since the library was loaded, left outputs to their second pass ([0]) and computed
+ * them again from fp32 operands ([1]; the others had nothing but zeros).  Waits for the device.
+ * 0 / -1. */
 int ptd_debug_conv_stats(uint64_t out[2]);
 int ptd_h2d(pt_ctx *c, void *dst, const void *src, size_t bytes);   /* synchronous */
 int ptd_d2h(pt_ctx *c, void *dst, const void *src, size_t bytes);   /* synchronous */

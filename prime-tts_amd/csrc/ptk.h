@@ -146,7 +146,7 @@ typedef struct {
 
 /* Relayout packed conv/convT weights [M/4][K][cin][4] into what the conv kernel reads
  * (ptk_kernels.hip, "weight relayout"): two fp16 parts of every weight, the fp32 weights, and a
- * factor per row, ptk_relayout_floats floats in all, 16-byte aligned.  ptk_conv_cinp: the channel
+ * factor and a threshold per row, ptk_relayout_floats floats in all, 16-byte aligned.  ptk_conv_cinp: the channel
  * count the kernel expects for this cin. */
 int ptk_conv_cinp(int cin);
 size_t ptk_relayout_floats(int M, int K, int cin);
@@ -164,9 +164,9 @@ int ptk_h2f(float *dst, const uint16_t *src, int64_t n, void *s);
 int ptk_conv_launch(const ptk_conv_desc *d, int ngroup, void *s);
 /* 1 when the MFMA kernel covers this problem's shape; else the caller uses the SIMT path */
 int ptk_conv_mfma_ok(const ptk_conv_desc *d);
-/* workgroups of the conv kernel, on the current device since the library was loaded, that looked at
- * their columns one by one, and that computed some of them again from fp32 operands; waits for the
- * device */
+/* workgroups of the conv kernel, on the current device since the library was loaded, that left
+ * outputs to their second pass, and that computed them again from fp32 operands (the others had
+ * nothing but zeros); waits for the device */
 int ptk_conv_stats(uint64_t out[2]);
 
 /* SIMT fallbacks over the PACKED layouts, for narrow shapes (cout4 < 16, tiny cin, huge K*dil):

@@ -357,11 +357,17 @@ extern "C" int ptk_graph_destroy(void *exec) {
 // The conv kernel multiplies fp32 operands on the fp16 matrix cores: an operand v, scaled by a
 // power of two into fp16's range, is taken as two fp16 parts
 //     hi = fp16(v),  lo = fp16(v - hi),
-// each rounded to nearest even (v - hi is exact in fp32).  hi + lo differs from v by at most 2^-24
-// of it while lo stays a normal fp16, half a unit in fp32's last place, and by 2^-25 absolute below
-// that.  Weights are scaled row by row so that the row's largest magnitude lies in [2^14, 2^15):
-// the absolute part is then 2^-39 of the row's largest weight.  Inputs take the fixed scale
-// 2^CONV_XS (see conv_mfma_kernel for the columns whose inputs do not fit).
+// each rounded to nearest even (v - hi is exact in fp32).  Together they hold 23 bits: hi + lo is
+// within 2^-23 of v while lo stays a normal fp16, and within half its smallest step below that.
+//   Weights are scaled row by row so that the row's largest magnitude lies in [2^14, 2^15): those
+//     below 2^-2 (2^-16 of the row's largest) are held to 2^-25 absolute.
+//   Inputs take the fixed scale 2^CONV_XS (up to 2^(16 - CONV_XS) fits), and their lo is stored times
+//     2^11, which puts its smallest step at 2^-35: inputs are held to 2^-36 absolute.
+// A product w x is summed as wl.xh + wh.xh + (wh 2^-11).(xl 2^11), the shifted wh formed in registers.
+// Dropping wl.xl costs up to 2^-22 of the product, so that one is within 2^-21 of w x (fp32: 2^-24),
+// plus the absolute parts: |w| 2^-35 from the input's side, |x| 2^-24 for a weight below 2^-2.
+// Whether those are small beside the products of an output is decided by conv_mfma_kernel with a
+// threshold per row that relayout_kernel makes.
 //
 // Packed [M/4][K][cin][4] (the reference's conv layout; a convT's phase rows are just more rows)
 // -> three parts, one after the other (Mp: M rounded up to 32, cinp: cin rounded up to 16; padding
@@ -373,9 +379,10 @@ extern "C" int ptk_graph_destroy(void *exec) {
 //     contiguous and so are the taps of its chunks.
 //   fp32 [Mp/32][cinp/16][K][64][8]: the weights themselves in the same order (conv_mfma_kernel's
 //     second pass).
-//   fp32 [Mp]: per row, the factor 2^-(row exponent + CONV_XS) that takes a sum of products of scaled
-//     operands back; NaN for a row that has no fp16 form (an inf or NaN weight, or all of it below
-//     2^-100).
+//   fp32 [2][Mp]: per row, the factor 2^-(row exponent + CONV_XS) that takes a sum of products of
+//     scaled operands back, and the threshold of that sum (see conv_mfma_kernel).  NaN and inf for a
+//     row that has no fp16 form (an inf or NaN weight, or all of it below 2^-100).
+//   fp32 [Mp/32]: the largest threshold of each row block.
 #define CONV_CK 16         // input channels per staged chunk (per wave)
 #define CONV_TAPB 2048     // bytes of one (row block, chunk, tap) of either copy of the weights
 // Waves per SIMD the registers are budgeted for, and (chunk, tap) slices the A operands are loaded
@@ -389,7 +396,10 @@ extern "C" int ptk_graph_destroy(void *exec) {
 #define CONV_LA1 2
 #define CONV_LA2 2
 #endif
-#define CONV_XS 6          // the inputs' scale, 2^CONV_XS
+// The inputs' scale, 2^CONV_XS: up to 2^12 an input fits its fp16 parts, and outputs of N(0, s) inputs
+// keep to the first pass down to about s = 2^-8 (a larger scale moves both ends down).
+#define CONV_XS 4
+#define CONV_LS 2048.0f    // the scale of the inputs' lo
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -397,7 +407,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 extern "C" int ptk_conv_cinp(int cin) { return (cin + CONV_CK - 1) / CONV_CK * CONV_CK; }
 extern "C" size_t ptk_relayout_floats(int M, int K, int cin) {
   const size_t Mp = (size_t) (M + 31) / 32 * 32;
-  return Mp * (size_t) K * (size_t) ptk_conv_cinp(cin) * 2 + Mp;
+  return Mp * (size_t) K * (size_t) ptk_conv_cinp(cin) * 2 + 2 * Mp + Mp / 32;
 }
 
 // two floats -> their fp16s (round to nearest even) in one word, a in the low half
@@ -405,12 +415,21 @@ __device__ __forceinline__ unsigned f16_pair(float a, float b) {
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
   return __builtin_bit_cast(unsigned, h2{(_Float16) a, (_Float16) b});
 }
-// the two parts of a pair of floats
+// the two parts of a pair of scaled weights
 __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &l) {
   const _Float16 ha = (_Float16) a, hb = (_Float16) b;
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
   h = __builtin_bit_cast(unsigned, h2{ha, hb});
   l = f16_pair(__builtin_fmaf((float) ha, -1.0f, a), __builtin_fmaf((float) hb, -1.0f, b));
+}
+// and of a pair of inputs, which it scales (exact: powers of two, and the fma's result is)
+__device__ __forceinline__ void split_input(float a, float b, unsigned &h, unsigned &l) {
+  constexpr float X = (float) (1 << CONV_XS);
+  const _Float16 ha = (_Float16) (a * X), hb = (_Float16) (b * X);
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  h = __builtin_bit_cast(unsigned, h2{ha, hb});
+  l = f16_pair(__builtin_fmaf((float) ha, -CONV_LS, a * (X * CONV_LS)),
+               __builtin_fmaf((float) hb, -CONV_LS, b * (X * CONV_LS)));
 }
 
 // Split planes: an activation tensor [C][T] already in two parts, scaled by 2^CONV_XS, as
@@ -427,11 +446,12 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsign
 #define RELAY_THREADS 256
 __global__ void __launch_bounds__(RELAY_THREADS) relayout_kernel(
     float *__restrict__ dst, const float *__restrict__ wp, int M, int K, int cin, int cinp, int il) {
-  __shared__ unsigned smax[4];
+  __shared__ unsigned smax[4], snum[4];
+  __shared__ unsigned long long sthr[4];
   const int Mp = (M + 31) / 32 * 32, nchunk = cinp / CONV_CK;
   const int tid = threadIdx.x, m0 = blockIdx.x * 4;
   const float4 *src = reinterpret_cast<const float4 *>(wp) + (long long) blockIdx.x * K * cin;
-  if (tid < 4) smax[tid] = 0;
+  if (tid < 4) smax[tid] = snum[tid] = 0, sthr[tid] = 0;
   __syncthreads();
   if (m0 < M) {
     unsigned mx[4] = {0, 0, 0, 0};   // as bit patterns: inf and NaN sort above every finite value
@@ -446,7 +466,7 @@ __global__ void __launch_bounds__(RELAY_THREADS) relayout_kernel(
     for (int r = 0; r < 4; r++) atomicMax(&smax[r], mx[r]);
   }
   __syncthreads();
-  float up[4];
+  float up[4], fac[4];
   int row[4];   // relaid rows
   const long long wn = (long long) Mp * K * cinp;
 #pragma unroll
@@ -459,9 +479,13 @@ __global__ void __launch_bounds__(RELAY_THREADS) relayout_kernel(
     const bool none = mx == 0, bad = !none && (e < -100 || mx >= 0x7f800000u);
     const int s = none || bad ? 0 : 14 - e;
     up[r] = __uint_as_float((unsigned) (127 + s) << 23);
-    if (tid == 0)
-      dst[2 * wn + row[r]] = bad ? __uint_as_float(0x7fc00000u) : __uint_as_float((unsigned) (127 - s - CONV_XS) << 23);
+    fac[r] = bad ? __uint_as_float(0x7fc00000u) : __uint_as_float((unsigned) (127 - s - CONV_XS) << 23);
+    if (tid == 0) dst[2 * wn + row[r]] = fac[r];
   }
+  // Of each row: the sum of its weights' magnitudes, each rounded up, plus 2^27 for every one below
+  // 2^-2 (integers: the same in any order), and the number of nonzero ones.
+  unsigned long long ta[4] = {0, 0, 0, 0};
+  unsigned nz[4] = {0, 0, 0, 0};
   for (int i = tid; i < nchunk * K * 2; i += RELAY_THREADS) {
     const int h = i & 1, k = (i >> 1) % K, chunk = (i >> 1) / K;
     float v[4][8];
@@ -480,6 +504,14 @@ __global__ void __launch_bounds__(RELAY_THREADS) relayout_kernel(
       const int lane = 32 * h + (row[r] & 31);
       u32x4 hi, lo;
 #pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const float m = fabsf(v[r][e] * up[r]);
+        if (m > 0.0f && m <= 32768.0f) {
+          nz[r]++;
+          ta[r] += (unsigned long long) (unsigned) ceilf(m) + (m < 0.25f ? 1ull << 27 : 0ull);
+        }
+      }
+#pragma unroll
       for (int e = 0; e < 4; e++) {
         unsigned a, b;
         split_pair(v[r][2 * e] * up[r], v[r][2 * e + 1] * up[r], a, b);
@@ -494,6 +526,29 @@ __global__ void __launch_bounds__(RELAY_THREADS) relayout_kernel(
       d32[1] = make_float4(v[r][4], v[r][5], v[r][6], v[r][7]);
     }
   }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    if (ta[r]) atomicAdd(&sthr[r], ta[r]);
+    if (nz[r]) atomicAdd(&snum[r], nz[r]);
+  }
+  __syncthreads();
+  if (tid < 4) {
+    // (sum |w| 2^-35 + 2^16 sum over the small ones of 2^-24) / (nonzero weights 2^-25): 0 for a row
+    // of zeros
+    const float f = tid == 0 ? fac[0] : tid == 1 ? fac[1] : tid == 2 ? fac[2] : fac[3];
+    const int rw = tid == 0 ? row[0] : tid == 1 ? row[1] : tid == 2 ? row[2] : row[3];
+    const float thr = snum[tid] ? (float) sthr[tid] * (1.0f / 1024) / (float) snum[tid] : 0.0f;
+    dst[2 * wn + Mp + rw] = f == f ? thr : __builtin_inff();
+  }
+}
+
+// the largest of the 32 thresholds of a row block; thr: the rows' thresholds, the results behind them
+__global__ void relayout_block_kernel(float *thr, int mt) {
+  const int mb = blockIdx.x * blockDim.x + threadIdx.x;
+  if (mb >= mt) return;
+  float m = 0.0f;
+  for (int r = 0; r < 32; r++) m = fmaxf(m, thr[mb * 32 + r]);
+  thr[mt * 32 + mb] = m;
 }
 
 static int relayout_il_ok(int M, int il, const char *who) {
@@ -508,6 +563,10 @@ extern "C" int ptk_relayout_il(float *dst, const float *wp, int M, int K, int ci
   if (!relayout_il_ok(M, il, "ptk_relayout_il")) return -1;
   hipLaunchKernelGGL(relayout_kernel, dim3((unsigned) ((M + 31) / 32 * 8)), dim3(RELAY_THREADS), 0,
                      (hipStream_t) s, dst, wp, M, K, cin, ptk_conv_cinp(cin), il);
+  HCHK(hipGetLastError());
+  const int mt = (M + 31) / 32;
+  hipLaunchKernelGGL(relayout_block_kernel, dim3((unsigned) ((mt + 63) / 64)), dim3(64), 0, (hipStream_t) s,
+                     dst + 2ll * (mt * 32) * K * ptk_conv_cinp(cin) + mt * 32, mt);
   HCHK(hipGetLastError());
   return 0;
 }
@@ -666,7 +725,7 @@ struct ConvGroup {
 #define CONV_NU_MAX 4
 // 16-byte LDS slots of one wave: its window / its partial sums
 static constexpr int conv_slots(int nu, int nb) { return nu * 32 * 4 > nb * 256 ? nu * 32 * 4 : nb * 256; }
-// and of the workgroup: one flag per wave, one magnitude per window column
+// and of the workgroup: flags, and one word per window column
 #define CONV_EXTRA_SLOTS (2 + CONV_NU_MAX * 8)
 
 // word 3 of a raw buffer resource on gfx9-family parts (gfx950): 32-bit data, range checked
@@ -692,46 +751,44 @@ struct Parts {
   f16x8 h, l;
 };
 
-// max(m, |a|, |b|); NaN if any of them is
-__device__ __forceinline__ float max_mag(float m, float a, float b) {
-  asm("v_maximum3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));
+// min(m, |a|, |b|); NaN if any of them is
+__device__ __forceinline__ float min_mag(float m, float a, float b) {
+  asm("v_minimum3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));
   return m;
 }
-__device__ __forceinline__ float half_of(unsigned pair, int i) {
-  return (float) __builtin_bit_cast(_Float16, (unsigned short) (pair >> (16 * i)));
-}
-// The largest input magnitude m of a receptive field for which the scaled fp16 parts hold the inputs
-// to 2^-24 of m: neither too large for fp16 nor so small that lo loses bits (all zero is exact).
-__device__ __forceinline__ bool conv_fits(float m) {
-  const float h = (float) (_Float16) (m * (float) (1 << CONV_XS));
-  return m == 0.0f || (h >= 0.25f && h <= 65504.0f);
-}
-// what the first pass tests on the fly: false wherever conv_fits is
-__device__ __forceinline__ bool conv_alarm_free(float m) {
-  return m < 1023.0f && (m >= 0.00390625f || m == 0.0f);
-}
 
-// Workgroups since the library was loaded that looked at their columns one by one / ran the second
-// pass (counted on those rare paths only).
+// Workgroups since the library was loaded that left outputs to the second pass / that ran it, the
+// others having found nothing but exact zeros (counted on those rare paths only).
 __device__ unsigned long long conv_stat[2];
 
 // One workgroup = S waves on one block of 32 rows x 32*NB columns.  The waves take disjoint runs of
 // the 16-channel chunks and are reduced through LDS in wave order (deterministic).  Each product of
-// two fp32 values is taken as three fp16 products on v_mfma_f32_32x32x16_f16 (hi.lo, lo.hi, hi.hi;
-// lo.lo is below 2^-24 of it), accumulated in fp32.
+// two fp32 values is taken as three fp16 products on v_mfma_f32_32x32x16_f16 (wl.xh, wh.xl, wh.xh:
+// "weight relayout" above), accumulated in fp32.
 //
-// An output column whose inputs (the receptive field, all channels) conv_fits refuses, and every
-// column of a row block with a weight that has no fp16 form, is computed by a second pass over the
-// block on v_mfma_f32_32x32x2_f32 instead, from the fp32 operands.  Which pass an output comes from
-// depends on its own receptive field only, not on the tile or batch it is computed in.  The first
-// pass watches the magnitudes it stages (a unit's own channels, so it may raise a false alarm but
-// misses nothing); only a workgroup it alarms looks at its columns one by one.
+// What an fp32 sum keeps is kept: with A = sum of |w x| over an output's products and n the nonzero
+// weights of its row, the operands' parts cost at most (n/2 + 8) 2^-24 A on top of the sum's own
+// rounding, whatever the magnitudes.  8 is the relative part.  The absolute parts, at most
+// sum |w| 2^-35 + 2^-8 per small weight in scaled units, have to be below n 2^-25 A.  A is at least the
+// sum over the waves of their partial sums' magnitudes: an output for which that is below its row's
+// threshold, or NaN (an input past 2^(16 - CONV_XS) makes it that, as inf and NaN do), is left over.
+// Ordinary outputs are not: all S partial sums would have to fall below about 2^-17 of their spread,
+// which for inputs N(0, s) some 1e-11 / s^2 of them do (S = 2, C 128, K 3).  Each wave looks at its
+// own partial sums first: in which eight rows of a column block is the smallest below the row block's
+// largest threshold?  Only a workgroup whose waves all name the same judges its outputs one by one,
+// one in a thousand of that launch.  (Judging every output and a barrier for the verdict took 0.3 us
+// of each launch.)
+//
+// Where outputs are left, the block is computed by a second pass on v_mfma_f32_32x32x2_f32, from the
+// fp32 operands, and they are stored from that: four rows of one lane together, so which pass an
+// output comes from depends on its own receptive field and the four rows' weights, not on the tile
+// or batch it is computed in.  Outputs that see nothing but zeros are left too, and skip that pass.
 //
 // Bound by the matrix cores on large launches (552 TFLOP/s of fp32 products at the rate the card
 // sustains, 150 on the fp32 matrix cores), by the way in and out of a workgroup on small ones.
 // Against the fp32-MFMA kernel it replaced: MRF-256 stack at T 904 149 -> 82 us, MRF-128 at T 3616
 // 154 -> 98 us, conv_pre at T 226 6.35 -> 5.6 us, ups.0 11.4 -> 9.5 us, a T 226 decode 345 -> 221 us
-// and eight in a batch 2141 -> 987 us; errors against 64 bits 0.6-0.8 of what they were.
+// and eight in a batch 2141 -> 987 us; errors against 64 bits 0.36-0.90 of what they were on N(0, 1).
 //
 // KT: the taps the straight-line bodies are built for (11: K = 11, 7 and 3; 4: K = 4, the convT
 // phase form); any other K goes through a rolled loop.  IN: input transform (PTK_IN_*).
@@ -744,7 +801,7 @@ conv_mfma_kernel(const ConvGroup g) {
   const int p = blockIdx.y;
   const ConvProb pi = g.info[p];
   // (a field of each scalar-cache line, so that all loads go out together, ahead of the test)
-  asm volatile("" ::"s"(pi.count), "s"(pi.x), "s"(pi.shift), "s"(pi.wslots));
+  asm volatile("" ::"s"(pi.count), "s"(pi.x), "s"(pi.nbias4), "s"(pi.shift), "s"(pi.bsx), "s"(pi.kd), "s"(pi.wslots), "s"(pi.ext_r));
   const int bid = blockIdx.x, wslots = pi.wslots;
   if (bid >= pi.count) return;
   // Tiles item after item, column tile after column tile, row block fastest: item 0 has its own
@@ -777,8 +834,6 @@ conv_mfma_kernel(const ConvGroup g) {
   // launcher refuses it elsewhere)
   const bool phase_il = KT == 4 && (pi.flags & PROB_PHASE_IL) != 0;
   const int r_tile = fdiv(mb, pi.div_phase);
-  // Every lane loads the scale of row lane & 31 of the block: NaN where a row has no fp16 form.
-  float scale_r = 0.0f;
   const int half = lane >> 5;     // which eight of a chunk's channels this lane feeds
   const int l32 = lane & 31;
   const int dmin = min(pi.kd, 0);
@@ -813,6 +868,7 @@ conv_mfma_kernel(const ConvGroup g) {
     }
   }
 
+  float thr_b = 0.0f;   // the row block's largest threshold
   // accumulators: one 32x32 block per column block (16 values per lane)
   f32x16 acc[NB];
 #pragma unroll
@@ -850,22 +906,15 @@ conv_mfma_kernel(const ConvGroup g) {
   // to six VALU instructions each (measured: 12 MFMAs 181 ns, with 72 VALU between them 185 ns), and
   // only the LDS stores stand between two chunks.  Rows past cin exist only when cin is not a
   // multiple of 16; MASK (compile time) selects the code that handles them.
-  bool odd = false;   // a magnitude conv_fits refuses was staged by this lane
   auto run = [&](auto kc, auto mask, auto nuc) {
     constexpr int KC = decltype(kc)::value, NU = decltype(nuc)::value;
     constexpr bool MASK = decltype(mask)::value;
     constexpr int PS = NU * 32;   // plane stride (16-byte slots)
     constexpr int PDM = NB == 1 ? CONV_PD1 : CONV_PD2, PD = KC == 0 ? 1 : KC < PDM ? KC : PDM;   // slices A is loaded ahead
     constexpr bool SPLIT = IN == PTK_IN_SPLIT;
-    float raw[NU][8], mag[NU];      // fp32 input: what is loaded, its largest magnitude
+    float raw[NU][8];               // fp32 input: what is loaded
     u32x4 raws[NU][2];              // split planes: what is loaded
-    unsigned hmax[NU], hmin[NU];    // and the extremes of its hi parts, pairwise
     u32x4 sp[NU][2];
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      mag[u] = 0.0f;
-      hmax[u] = hmin[u] = 0;
-    }
     auto load_unit = [&](__amdgpu_buffer_rsrc_t rx, int u, int j) {
       const int ci0 = (chunk0 + j) * CONV_CK;
       if constexpr (SPLIT) {
@@ -889,16 +938,11 @@ conv_mfma_kernel(const ConvGroup g) {
       if constexpr (SPLIT) {
         sp[u][0][e] = raws[u][0][e];
         sp[u][1][e] = raws[u][1][e];
-        if (e & 1) {
-          asm("v_pk_maximum3_f16 %0, %1, %2, %0" : "+v"(hmax[u]) : "v"(raws[u][0][e - 1]), "v"(raws[u][0][e]));
-          asm("v_pk_minimum3_f16 %0, %1, %2, %0" : "+v"(hmin[u]) : "v"(raws[u][0][e - 1]), "v"(raws[u][0][e]));
-        }
         return;
       }
       const float a = in_xform<IN>(raw[u][2 * e], in_a), b = in_xform<IN>(raw[u][2 * e + 1], in_a);
       unsigned h, l;
-      mag[u] = max_mag(mag[u], a, b);
-      split_pair(a * (float) (1 << CONV_XS), b * (float) (1 << CONV_XS), h, l);
+      split_input(a, b, h, l);
       sp[u][0][e] = h;
       sp[u][1][e] = l;
     };
@@ -921,8 +965,8 @@ conv_mfma_kernel(const ConvGroup g) {
       q.l = __builtin_bit_cast(f16x8, xr[2 * PS]);
       return q;
     };
-    auto mfma3 = [&](const Parts &a, const Parts &c, int nb) {
-      acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.h, c.l, acc[nb], 0, 0, 0);
+    auto mfma3 = [&](const Parts &a, const f16x8 &hs, const Parts &c, int nb) {
+      acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hs, c.l, acc[nb], 0, 0, 0);
       acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.l, c.h, acc[nb], 0, 0, 0);
       acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.h, c.h, acc[nb], 0, 0, 0);
     };
@@ -933,7 +977,10 @@ conv_mfma_kernel(const ConvGroup g) {
     for (int u = 0; u < NU; u++) load_unit(rx, u, 0);
 #pragma unroll
     for (int k = 0; k < PD; k++) ahead[k] = wa(rw, min(k, last));
-    scale_r = pi.scale[mb * 32 + l32];
+    // (a vector load, in line behind those that the loop waits for; a scalar one would hold up its
+    // first LDS reads)
+    thr_b = buf_load(__builtin_amdgcn_make_buffer_rsrc((void *) (pi.scale + pi.mt * 64), (short) 0, pi.mt * 4, PTK_BUF_WORD3), 0,
+                     (unsigned) mb * 4u);
     {
       const __amdgpu_buffer_rsrc_t rx1 = x_rsrc(nch > 1);
 #pragma unroll
@@ -956,6 +1003,7 @@ conv_mfma_kernel(const ConvGroup g) {
         for (int k = 0; k < PD; k++) a[k] = ahead[k];
         constexpr int LA = NB == 1 ? CONV_LA1 : CONV_LA2;   // steps the B operands are read ahead
         Parts q[NS + LA];
+        f16x8 hs;   // a[k].h shifted to the lo's scale
 #pragma unroll
         for (int s = 0; s < LA; s++) q[s] = col(s / NB, s % NB);
 #pragma unroll
@@ -970,7 +1018,8 @@ conv_mfma_kernel(const ConvGroup g) {
               split_unit(i / 4, i % 4);
               if (i % 4 == 3) load_unit(rx2, i / 4, j + 2);
             }
-          mfma3(a[k], q[s], nb);
+          if (nb == 0) hs = a[k].h * (_Float16) (1.0f / CONV_LS);
+          mfma3(a[k], hs, q[s], nb);
           __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
@@ -981,7 +1030,7 @@ conv_mfma_kernel(const ConvGroup g) {
           ahead[0] = wa(rw, min(j * K + k + 1, last));
           PTK_PIN_VMEM();
 #pragma unroll
-          for (int nb = 0; nb < NB; nb++) mfma3(a, col(k, nb), nb);
+          for (int nb = 0; nb < NB; nb++) mfma3(a, a.h * (_Float16) (1.0f / CONV_LS), col(k, nb), nb);
         }
 #pragma unroll
         for (int u = 0; u < NU; u++) {
@@ -991,56 +1040,67 @@ conv_mfma_kernel(const ConvGroup g) {
         }
       }
     }
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      if constexpr (SPLIT) {   // all zero alarms too: an input too small for hi and lo looks like that
-        const float m = max_mag(max_mag(0.0f, half_of(hmax[u], 0), half_of(hmax[u], 1)),
-                                half_of(hmin[u], 0), half_of(hmin[u], 1));
-        odd |= voff[u] != PTK_OOB && !(m <= 65504.0f && m >= 0.25f);
-      } else {
-        odd |= !conv_alarm_free(mag[u]);
-      }
-    }
   };
-  // The second pass: the same chunks from fp32 operands, in one rolled loop.  The window is staged
-  // as planes [h][e >> 2] of float4 columns (channels 8h + e): the same LDS.
+  // The second pass: the same chunks from fp32 operands, in one rolled loop; the loads of a chunk's
+  // window go out ahead of the taps of the chunk before it, those of a tap's weights ahead of the tap
+  // before it.  The window is staged as planes [h][e >> 2] of float4 columns (channels 8h + e): the
+  // same LDS.  pi, p: the launch facts, read again (kept from the first pass they would take the
+  // scalar registers of the common path).
   // the input transform as the fp32 operands need it: split planes hold LeakyReLU(in_a) of d.x
-  auto xform32 = [&](float v) {
-    return in_xform<IN == PTK_IN_PLAIN ? PTK_IN_PLAIN : PTK_IN_LEAKY>(v, in_a);
+  auto xform32 = [&](float v, float a) {
+    return in_xform<IN == PTK_IN_PLAIN ? PTK_IN_PLAIN : PTK_IN_LEAKY>(v, a);
   };
-  auto run32 = [&](const ptk_conv_desc &d) {
-    const int PS = g.wcols;
+  auto run32 = [&](const ConvProb &pi, int p) {
+    const ptk_conv_desc &d = g.d[p];
+    const int PS = g.wcols, K = pi.K, dil = pi.dil, st = pi.st, cin = pi.cin, nchunk = pi.nchunk;
+    const unsigned ldx4 = (unsigned) pi.ldx4;
+    const float in_a = pi.in_a;
+    const int chunk0 = w * nchunk / S, nch = (w + 1) * nchunk / S - chunk0;
+    if (nch == 0) return;
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-        (void *) (d.x + xoff), (short) 0, (int) nrec, PTK_BUF_WORD3);
+        (void *) (d.x + b * pi.bsx), (short) 0, (int) ((unsigned) cin * ldx4), PTK_BUF_WORD3);
     const float4 *const wr = reinterpret_cast<const float4 *>(d.w + (long long) (pi.mt * 32) * K * d.cinp) +
                              ((long long) mb * nchunk + chunk0) * K * (CONV_TAPB / 16) + lane * 2;
     float4 *const x4 = reinterpret_cast<float4 *>(xs);
-    for (int j = 0; j < nch; j++) {
+    float raw[CONV_NU_MAX][8];
+    auto load = [&](int j) {
       const int ci0 = (chunk0 + j) * CONV_CK + 8 * half;
+#pragma unroll
+      for (int u = 0; u < CONV_NU_MAX; u++) {
+        if (32 * u >= PS) continue;
+        const unsigned c4 = IN == PTK_IN_SPLIT ? (voff[u] - (unsigned) (8 * half) * ldx4) / 4u
+                                               : voff[u] - (unsigned) (8 * half) * ldx4;
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          raw[u][e] = buf_load(rx, j < nch && voff[u] != PTK_OOB && ci0 + e < cin
+                                       ? c4 + (unsigned) (ci0 + e) * ldx4 : PTK_OOB, 0);
+      }
+    };
+    load(0);
+    float4 a0 = wr[0], a1 = wr[1];
+    for (int j = 0; j < nch; j++) {
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int u = 0; u < CONV_NU_MAX; u++) {
         if (32 * u >= PS) continue;
         float v[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const unsigned c4 = IN == PTK_IN_SPLIT ? (voff[u] - (unsigned) (8 * half) * ldx4) / 4u
-                                                 : voff[u] - (unsigned) (8 * half) * ldx4;
-          v[e] = xform32(buf_load(rx, voff[u] != PTK_OOB && ci0 + e < cin
-                                          ? c4 + (unsigned) (ci0 + e) * ldx4 : PTK_OOB, 0));
-        }
+        for (int e = 0; e < 8; e++) v[e] = xform32(raw[u][e], in_a);
         x4[2 * half * PS + 32 * u + l32] = make_float4(v[0], v[1], v[2], v[3]);
         x4[(2 * half + 1) * PS + 32 * u + l32] = make_float4(v[4], v[5], v[6], v[7]);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      load(j + 1);
+      PTK_PIN_VMEM();
       for (int k = 0; k < K; k++) {
-        const float4 *const wk = wr + (long long) (j * K + k) * (CONV_TAPB / 16);
-        const float4 a0 = wk[0], a1 = wk[1];
+        const float4 *const wk = wr + (long long) min(j * K + k + 1, nch * K - 1) * (CONV_TAPB / 16);
+        const float4 n0 = wk[0], n1 = wk[1];
+        PTK_PIN_VMEM();
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) {
-          const float4 *const xr = x4 + 2 * half * PS + (l32 + 32 * nb) * st - dmin + k * dil;
+          const float4 *const xr = x4 + 2 * half * PS + (l32 + 32 * nb) * st - min((K - 1) * dil, 0) + k * dil;
           const float4 b0 = xr[0], b1 = xr[PS];
           acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, b0.x, acc[nb], 0, 0, 0);
           acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, b0.y, acc[nb], 0, 0, 0);
@@ -1051,6 +1111,8 @@ conv_mfma_kernel(const ConvGroup g) {
           acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.z, b1.z, acc[nb], 0, 0, 0);
           acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.w, b1.w, acc[nb], 0, 0, 0);
         }
+        a0 = n0;
+        a1 = n1;
       }
     }
   };
@@ -1060,7 +1122,7 @@ conv_mfma_kernel(const ConvGroup g) {
   const bool narrow = XW <= 32 * (NB + 1);
   // channel padding in the last chunk, a stride or another K: the rolled body
   const int straight = cin == nchunk * CONV_CK && st == 1 ? K : 0;
-  if (nch == 0) scale_r = pi.scale[mb * 32 + l32];
+  if (nch == 0) {}
   else if (KT == 4 && straight == 4 && narrow) run(std::integral_constant<int, KT == 4 ? 4 : 0>{}, nomask, few);
   else if (KT == 11 && straight == 11 && narrow) run(std::integral_constant<int, KT == 11 ? 11 : 0>{}, nomask, few);
   else if (KT == 11 && straight == 11) run(std::integral_constant<int, KT == 11 ? 11 : 0>{}, nomask, all);
@@ -1076,16 +1138,18 @@ conv_mfma_kernel(const ConvGroup g) {
   const int v0 = w * NMAX;
   const int addt = pi.addt;   // the chain's residual add, if any
   auto vrow = [&](int i) { return 8 * ((v0 + i) >> 2) + 4 * half + ((v0 + i) & 3); };   // of value i
-  unsigned mine = ~0u;   // bit nb: this pass stores the lane's column of block nb
-  bool again = false;    // some column is left to the second pass
+  // bit nb * NG + gg: outputs of group gg, column block nb, that the first pass leaves
+  unsigned left = 0;
+  int *const flags = reinterpret_cast<int *>(smem + S * wslots);
+  bool nonzero = false;   // some partial sum of theirs is not zero, or their row has no fp16 form
+  bool judged = false;    // the workgroup judged its outputs
   // (once for each pass, not a loop over them: the compiler would compute everything the rare paths
   // need ahead of the loop, some 200 instructions)
-  auto finish = [&](auto passc) {
+  auto finish = [&](auto passc, const ConvProb &pi, int p) {
   constexpr int pass = decltype(passc)::value;
   const ptk_conv_desc &d = g.d[p];
   // Each wave writes its partial sums over its own staging area, which only it reads, so no wave
   // waits for the others before writing: [nb][v >> 2][lane] float4.
-  int *const flags = reinterpret_cast<int *>(smem + S * wslots);
   {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     f32x4 *red = reinterpret_cast<f32x4 *>(xs);
@@ -1099,38 +1163,73 @@ conv_mfma_kernel(const ConvGroup g) {
         red[(nb * 4 + q) * 64 + lane] = v;
       }
   }
-  const bool alarm = pass == 0 && __ballot(odd || scale_r != scale_r) != 0;
-  if (pass == 0 && lane == 0) flags[w] = alarm;
-  // the barrier behind the partial sums; then, in a workgroup that was alarmed, the columns that
-  // are left to the second pass
+  // A wave's look at its own partial sums (while the epilogue's loads are on their way) and the barrier
+  // behind them.  Returns what the waves say, read together with the first sums.
   auto reduce_wait = [&]() {
-    __syncthreads();
-    if (pass != 0) return;
-    int any = flags[0];
-#pragma unroll
-    for (int i = 1; i < S; i++) any |= flags[i];
-    if (__builtin_expect(__builtin_amdgcn_readfirstlane(any) == 0, 1)) return;
-    if (threadIdx.x == 0) atomicAdd(&conv_stat[0], 1ull);
-    float *const cm = reinterpret_cast<float *>(smem + S * wslots + 2);   // per window column
-    for (int i = threadIdx.x; i < XW; i += 64 * S) {
-      const int c = cmin + i, pc = pi.flags & PROB_REFLECT ? (c == 0 ? 1 : c - 1) : c;
-      float m = 0.0f;
-      if (c >= 0 && c < cend)
-        for (int ci = 0; ci < cin; ci++) m = max_mag(m, xform32(d.x[xoff + (long long) ci * d.ldx + pc]), 0.0f);
-      cm[i] = m;
+    if (pass != 0) {
+      __syncthreads();
+      return 0;
     }
-    __syncthreads();
-    const bool bad_w = __ballot(scale_r != scale_r) != 0;
-    const long long qend = d.q0 + d.nq + (last_item ? d.ext_r : 0);
-    mine = 0;
+    const int qend = pi.qend + (last_item ? pi.ext_r : 0);
+    unsigned low = 0;   // bit 4 * nb + (v >> 2): rows 8 * (v >> 2) .. + 7 of column block nb
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
-      float m = 0.0f;
-      for (int k = 0; k < K; k++) m = max_mag(m, cm[(l32 + 32 * nb) * st - dmin + k * dil], 0.0f);
-      // (a column past the end is stored by neither pass)
-      if (q0 + 32 * nb + l32 >= qend || (!bad_w && conv_fits(m))) mine |= 1u << nb;
+      const unsigned long long used = __ballot(q0 + 32 * nb + l32 < qend);
+#pragma unroll
+      for (int v = 0; v < 16; v += 4) {
+        const float m = min_mag(min_mag(__builtin_inff(), acc[nb][v], acc[nb][v + 1]), acc[nb][v + 2], acc[nb][v + 3]);
+        low |= (__ballot(!(m >= thr_b)) & used) != 0 ? 1u << (4 * nb + v / 4) : 0u;
+      }
     }
-    again = __ballot(mine != (1u << NB) - 1) != 0;
+    const int rows = pi.M - mb * 32;   // (the padding rows behind them are all zero)
+    low &= rows >= 32 ? 0xffu : 0x11u * ((1u << ((rows + 7) >> 3)) - 1);
+    if (low != 0) {   // a NaN makes the workgroup judge whatever the other waves have
+      float m = 0.0f;
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+        for (int v = 0; v < 16; v += 2) m = min_mag(m, acc[nb][v], acc[nb][v + 1]);
+      if (__ballot(m != m) != 0) low |= 0x100;
+    }
+    if (lane == 0) flags[w] = nch > 0 ? (int) low : 0xff;   // (a wave without channels has no say)
+    if (threadIdx.x == 0) flags[4] = flags[5] = 0;
+    __syncthreads();
+    int all = flags[0], nan = all;
+#pragma unroll
+    for (int i = 1; i < S; i++) {
+      all &= flags[i];
+      nan |= flags[i];
+    }
+    return all | (nan & 0x100);
+  };
+  // The judging, if all waves ask for it.
+  auto judge = [&](int say) {
+    if (pass != 0 || __builtin_expect(__builtin_amdgcn_readfirstlane(say) == 0, 1)) return;
+    judged = true;
+    const int qend = pi.qend + (last_item ? pi.ext_r : 0);
+    f32x4 thr[NG];
+#pragma unroll
+    for (int gg = 0; gg < NG; gg++)
+      thr[gg] = *reinterpret_cast<const f32x4 *>(pi.scale + (pi.mt + mb) * 32 + vrow(gg * GRP));
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+      for (int gg = 0; gg < NG; gg++) {
+        f32x4 m = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < S; i++)
+          m += __builtin_elementwise_abs(reinterpret_cast<const f32x4 *>(smem + i * wslots)[(nb * 4 + (v0 >> 2) + gg) * 64 + lane]);
+        bool ok = true, some = false;
+#pragma unroll
+        for (int e = 0; e < GRP; e++) {
+          const bool is = m[e] >= thr[gg][e] && m[e] < __builtin_inff();
+          ok &= is;
+          some |= !is && (m[e] != 0.0f || thr[gg][e] == __builtin_inff());
+        }
+        const bool used = q0 + 32 * nb + l32 < qend;
+        left |= (unsigned) (used && !ok) << (nb * NG + gg);
+        nonzero |= used && some;
+      }
   };
   // The S partial sums of a group's values, in wave order.
   auto reduced = [&](int nb, int gg) {
@@ -1198,12 +1297,12 @@ conv_mfma_kernel(const ConvGroup g) {
         else scale[gg] = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
       }
     }
-    reduce_wait();
+    const int say = reduce_wait();
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
       const int q = q0 + 32 * nb + l32;
       const int col = q * ep.ys + r_tile - ep.ypad;   // phase_il: the sample of phase 0 (r_tile = 0)
-      const bool oq = q < qend32 && (mine >> nb & 1);
+      const bool oq = q < qend32;
       float val[NMAX];
 #pragma unroll
       for (int gg = 0; gg < NG; gg++) {
@@ -1211,6 +1310,7 @@ conv_mfma_kernel(const ConvGroup g) {
 #pragma unroll
         for (int i = 0; i < GRP; i++) val[gg * GRP + i] = fmaf(sum[i], scale[gg][i], bias[gg][i]);
       }
+      if (nb == 0) judge(say);
       // The chain.  The decoder's two chains, a LeakyReLU and a tensor add (the chain's one, the
       // launcher's rule), have their own code; any other goes op by op.
       if (ep.ops == PTK_EPI_ADDT) {
@@ -1233,14 +1333,14 @@ conv_mfma_kernel(const ConvGroup g) {
           }
         }
       }
-      // Stores by groups: four (or two) rows of one v >> 2.  Rows interleaved by phase: v >> 2 is
+      // Stores by groups: four rows of one v >> 2.  Rows interleaved by phase: v >> 2 is
       // the phase, the column's sample.
 #pragma unroll
       for (int gg = 0; gg < NG; gg++) {
         const int vg = v0 + gg * GRP;
         const int cg = phase_il ? col + (vg >> 2) : col;
         const int rg = phase_il ? (vg & 3) : urow(gg * GRP);   // uniform part of the group's first row
-        if (!(oq && cg >= 0 && cg < ep.lout)) continue;
+        if (!(oq && cg >= 0 && cg < ep.lout && (left >> (nb * NG + gg) & 1) == pass)) continue;
         const unsigned vo = (unsigned) (4 * half * ldy32 + cg) * 4u;
 #pragma unroll
         for (int i = 0; i < GRP; i++) {
@@ -1256,8 +1356,7 @@ conv_mfma_kernel(const ConvGroup g) {
 #pragma unroll
           for (int i = 0; i < GRP; i += 2) {
             const float a = val[gg * GRP + i], c = val[gg * GRP + i + 1];
-            split_pair((a >= 0.0f ? a : ep.a2 * a) * (float) (1 << CONV_XS),
-                       (c >= 0.0f ? c : ep.a2 * c) * (float) (1 << CONV_XS), h[i / 2], l[i / 2]);
+            split_input(a >= 0.0f ? a : ep.a2 * a, c >= 0.0f ? c : ep.a2 * c, h[i / 2], l[i / 2]);
           }
           const unsigned vs = (unsigned) cg * 16u + (unsigned) half * 8u;
           const unsigned ss = (unsigned) ((rg >> 3) * 8 * ldy32) * 4u + (unsigned) (rg & 3) * 2u;
@@ -1278,7 +1377,7 @@ conv_mfma_kernel(const ConvGroup g) {
   const float a2 = d.a2;
   const bool phase_rows = C4 != M;
   const long long qend = d.q0 + d.nq + (last_item ? d.ext_r : 0);
-  reduce_wait();
+  judge(reduce_wait());
 #pragma unroll 1
   for (int nb = 0; nb < NB; nb++) {
     const long long q = (long long) q0 + 32 * nb + l32;
@@ -1288,7 +1387,7 @@ conv_mfma_kernel(const ConvGroup g) {
 #pragma unroll
     for (int i = 0; i < GRP; i++) {
       const int m = mb * 32 + vrow(gg * GRP + i);
-      if (m >= M || q >= qend || !(mine >> nb & 1)) continue;
+      if (m >= M || q >= qend || (left >> (nb * NG + gg) & 1) != pass) continue;
       int co = m, r = 0;
       if (phase_il) {
         r = (m >> 3) & 3;
@@ -1307,7 +1406,7 @@ conv_mfma_kernel(const ConvGroup g) {
       if (y2b != nullptr) y2b[yi] = vl;
       if (ysb != nullptr) {
         unsigned h, l;
-        split_pair(vl * (float) (1 << CONV_XS), 0.0f, h, l);
+        split_input(vl, 0.0f, h, l);
         unsigned short *const ys16 = reinterpret_cast<unsigned short *>(ysb + (long long) (co & ~7) * ldy) + col * 8 + (co & 7);
         ys16[0] = (unsigned short) h;
         ys16[8 * ldy] = (unsigned short) l;
@@ -1317,18 +1416,56 @@ conv_mfma_kernel(const ConvGroup g) {
   }
   }
   };
-  finish(std::integral_constant<int, 0>{});
-  if (__builtin_expect(!again, 1)) return;
-  // the columns left over, from fp32 operands
-  if (threadIdx.x == 0) atomicAdd(&conv_stat[1], 1ull);
-  mine = ~mine;
+  finish(std::integral_constant<int, 0>{}, pi, p);
+  if (__builtin_expect(!judged, 1)) return;
+  if (left) flags[4] = 1;
+  if (nonzero) flags[5] = 1;
+  __syncthreads();   // (every wave is done with the first pass's partial sums, too)
+  if (__builtin_amdgcn_readfirstlane(flags[4]) == 0) return;
+  if (threadIdx.x == 0) atomicAdd(&conv_stat[0], 1ull);
+  int p2 = blockIdx.y;
+  asm volatile("" : "+s"(p2));   // (so that the facts are read again, see run32)
+  const ConvProb pr = g.info[p2];
+  int again = __builtin_amdgcn_readfirstlane(flags[5]);
+  if (again == 0) {
+    // Sums of exactly zero: of nothing but zeros, or of values below the parts' range?  Threads take a
+    // column each and share its channels.
+    const ptk_conv_desc &d = g.d[p2];
+    const int XW = pr.xw, K = pr.K, dil = pr.dil, st = pr.st, cin = pr.cin;
+    const int dmin = min(pr.kd, 0), cmin = q0 * st + dmin - pr.shift;
+    const int cend = min(pr.lim, (min(q0 + 32 * NB, pr.qend + (last_item ? pr.ext_r : 0)) - 1) * st + max(pr.kd, 0) - pr.shift + 1);
+    int *const cm = flags + 8;   // per window column: it holds something
+    const int cols = XW <= 64 ? 64 : 128, i = threadIdx.x & (cols - 1);
+    for (int k = threadIdx.x; k < 32 * CONV_NU_MAX; k += 64 * S) cm[k] = 0;
+    __syncthreads();
+    const int c = cmin + i, pc = pr.flags & PROB_REFLECT ? (c == 0 ? 1 : c - 1) : c;
+    if (i < XW && c >= 0 && c < cend) {
+      bool any = false;
+#pragma unroll 8
+      for (int ci = threadIdx.x / cols; ci < cin; ci += 64 * S / cols)
+        any |= xform32(d.x[b * pr.bsx + (long long) ci * d.ldx + pc], pr.in_a) != 0.0f;
+      if (any) cm[i] = 1;
+    }
+    __syncthreads();
+    int seen = 0;
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++)
+      if (left >> (nb * NG) & ((1u << NG) - 1))
+        for (int k = 0; k < K; k++) seen |= cm[(l32 + 32 * nb) * st - dmin + k * dil];
+    if (seen) flags[5] = 1;
+    __syncthreads();
+    again = __builtin_amdgcn_readfirstlane(flags[5]);
+  }
+  // the outputs left over, from fp32 operands (zeros add up to what the first pass has: zero)
 #pragma unroll
   for (int nb = 0; nb < NB; nb++)
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[nb][v] = 0.0f;
-  __syncthreads();   // every wave is done with the first pass's partial sums
-  if (nch > 0) run32(g.d[p]);
-  finish(std::integral_constant<int, 1>{});
+  if (again) {
+    if (threadIdx.x == 0) atomicAdd(&conv_stat[1], 1ull);
+    run32(pr, p2);
+  }
+  finish(std::integral_constant<int, 1>{}, pr, p2);
 }
 
 static int conv_window(const ptk_conv_desc *d, int nb) {
@@ -2081,7 +2218,7 @@ __global__ void __launch_bounds__(128) avg3_leaky_split_kernel(
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       unsigned hh, ll;
-      split_pair(v[2 * e] * (float) (1 << CONV_XS), v[2 * e + 1] * (float) (1 << CONV_XS), hh, ll);
+      split_input(v[2 * e], v[2 * e + 1], hh, ll);
       h[e] = hh;
       l[e] = ll;
     }

@@ -1,11 +1,11 @@
-"""The conv kernel's two passes: products of fp32 operands as fp16 parts for inputs whose magnitudes
-the parts hold (2^-8 to 1023 in a receptive field), from the fp32 operands for every other column.
+"""The conv kernel's two passes: products of fp32 operands as fp16 parts for the outputs whose sums
+are large enough beside what the parts round off, from the fp32 operands for every other output.
 
-The bar on values is the bound of an fp32 sum in any order, |err| <= n 2^-24 sum |w x| over the n
-products of an output (float64 reference), at every input scale: columns of inputs far below 2^-8
-meet it only if they are left to the second pass, whose operands are the fp32 ones, and those past
-1023 are infinite in the first.  Which pass a column comes from depends on its own inputs only, so
-a column that does not see a disturbance keeps its bits."""
+The bar on values is componentwise, |err| <= c n 2^-24 sum |w x| over the n products of an output
+(float64 reference): an fp32 sum in any order keeps to it with c = 1, the parts add n/2 + 8 of the
+same.  It holds at every input scale and for any mix of magnitudes, among the inputs of an output and
+among the weights of a row.  Which pass an output comes from depends on its own inputs and its rows'
+weights, so a column that does not see a disturbance keeps its bits."""
 from __future__ import annotations
 
 import ctypes as C
@@ -177,3 +177,86 @@ def test_layer_alone_equals_layer_in_a_decode():
         d.free()
     model.close()
     ctx.close()
+
+
+# mixes of magnitudes: inputs by channel, weights by element, weights that undo the inputs' scales,
+# and rows that select one quiet channel beside loud ones
+def _mixed(kind, rng, x, W):
+    cout, cin, K = W.shape
+    if kind == "inputs":
+        return x * 10.0 ** rng.uniform(-30, 3, (cin, 1)), W
+    if kind == "weights":
+        return x, W * 10.0 ** rng.uniform(-12, 6, W.shape)
+    if kind == "opposed":
+        s = 10.0 ** rng.uniform(-8, 3, (cin, 1))
+        return x / s, W * s
+    W = np.zeros_like(W)
+    for m in range(cout):
+        W[m, (5 * m) % cin, m % K] = 1.0
+        if m % 4 == 1:
+            W[m, (5 * m + 1) % cin, m % K] = 1e-6   # beside a weight far below the row's largest
+    return x * 10.0 ** rng.uniform(-14, 2, (cin, 1)), W
+
+
+@pytest.mark.parametrize("cin,K,dil,stride", SHAPES)
+@pytest.mark.parametrize("kind", ["inputs", "weights", "opposed", "select"])
+@pytest.mark.parametrize("split,nb", [(0, 0), (2, 1), (2, 2), (4, 1), (4, 2)])
+def test_mixed_magnitudes_meet_the_componentwise_bound(ctx, cin, K, dil, stride, kind, split, nb, knob_env):
+    """|err| <= (n + n/2 + 9) 2^-24 sum |w x|, n the nonzero weights of the row: the sum's own rounding
+    and the bias, and the parts'.  On every tile shape."""
+    if split:
+        knob_env.setenv("PTK_CONV_SPLIT", str(split))
+        knob_env.setenv("PTK_CONV_NB", str(nb))
+    rng, x, W, _ = case(cin, 72, K, 150, seed=7)
+    x, W = _mixed(kind, rng, x, W)
+    x, W, b = x.astype(np.float32), W.astype(np.float32), np.zeros(72, np.float32)
+    pad = (K - 1) * dil // 2
+    y = gpu_conv(ctx, x, synth.pack_conv(W), b, 72, K, stride, pad, dil)[:, :72]
+    ref, mag = conv64(x, W, b, pad, dil, stride)
+    n = np.count_nonzero(W, axis=(1, 2))[:, None]
+    tiny = n * 2.0 ** -149   # products below fp32's range
+    assert np.all(np.abs(y - ref) <= (1.5 * n + 9) * 2.0 ** -24 * mag + tiny)
+
+
+def test_examples_of_lost_range(ctx):
+    """One quiet input beside a loud one, one small weight beside a large one: exactly what fp32 gives
+    (a product with 1 is exact)."""
+    for q in (1e-6, 1e-7, 1e-10, 1e-30):
+        x = np.zeros((1, 16, 40), np.float32)
+        x[:, 0], x[:, 1] = 1.0, np.float32(q)
+        W = np.zeros((32, 16, 1), np.float32)
+        W[:, 1] = 1.0
+        y = gpu_conv(ctx, x, synth.pack_conv(W), np.zeros(32, np.float32), 32, 1, 1, 0, 1)
+        assert np.all(np.abs(y - np.float32(q)) <= 2.0 ** -21 * q), q
+    x[:, 1], W[:, 0], W[:, 1] = 1.1e-6, 1e-6, 1e6
+    y = gpu_conv(ctx, x, synth.pack_conv(W), np.zeros(32, np.float32), 32, 1, 1, 0, 1)
+    want = np.float64(np.float32(1e-6)) + np.float64(np.float32(1e6)) * np.float64(np.float32(1.1e-6))
+    assert np.all(np.abs(y - want) <= 12 * 2.0 ** -24 * want)
+
+
+def _stats(ctx):
+    n = (C.c_uint64 * 2)()
+    assert ctx.lib.ptd_debug_conv_stats(n) == 0
+    return np.array([n[0], n[1]])
+
+
+def test_ordinary_inputs_and_silence_stay_on_the_first_pass(ctx):
+    """N(0, 1) inputs leave no output to the second pass; columns of zeros, alone and next to sound,
+    leave theirs and find nothing to compute again: the bias, exactly."""
+    rng, x, W, b = case(192, 96, 7, 400, seed=3)
+    wp = synth.pack_conv(W)
+    n0 = _stats(ctx)
+    y0 = gpu_conv(ctx, x, wp, b, 96, 7, 1, 3, 1)
+    n1 = _stats(ctx)
+    assert not np.any(n1 - n0)
+    x[:, :, 100:300] = 0.0
+    y = gpu_conv(ctx, x, wp, b, 96, 7, 1, 3, 1)
+    n2 = _stats(ctx)
+    assert n2[0] > n1[0] and n2[1] == n1[1]
+    assert np.array_equal(y[:, :, 103:297], np.broadcast_to(b[:, None], y[:, :, 103:297].shape))
+    assert np.array_equal(y[:, :, :97], y0[:, :, :97]) and np.array_equal(y[:, :, 303:], y0[:, :, 303:])
+    x[0, 17, 200] = 1e-30   # below the parts' range: the second pass sees it
+    y = gpu_conv(ctx, x, wp, np.zeros(96, np.float32), 96, 7, 1, 3, 1)
+    assert _stats(ctx)[1] > n2[1]
+    want = np.float64(W[:, 17, ::-1]) * np.float64(x[0, 17, 200])
+    assert np.all(np.abs(y[0, :, 197:204] - want) <= 2.0 ** -23 * np.abs(want))
