@@ -272,26 +272,34 @@ def test_batched_decode_matches_single(env, T, batch):
     dz.free(); dw.free()
 
 
+def _force_tile(knob_env, split, nb):
+    if split:
+        knob_env.setenv("PTK_CONV_SPLIT", str(split))
+        knob_env.setenv("PTK_CONV_NB", str(nb))
+
+
 # (layer, T, cols relative to the full launch: q0 offset, nq, ext_l, ext_r)
 LAYER_COLS = [(0, 150, 20, 70, 13, 31), (1, 60, 9, 33, 5, 17), (20, 90, 30, 41, 29, 2),
               (18, 300, 37, 151, 36, 100), (37, 200, 100, 1, 99, 99), (38, 130, 1, 64, 0, 0),
               (39, 257, 64, 128, 40, 65)]
 
 
-@pytest.mark.parametrize("rb,split", [(0, 0), (16, 1), (32, 2), (32, 4), (16, 4), (16, 8), (32, 8)])
-def test_layer_cols_per_item(env, rb, split, knob_env):
+# (channel split, column blocks per wave); (0, 0): the launcher's choice
+TILES = [(0, 0), (2, 1), (2, 2), (4, 1), (4, 2)]
+
+
+@pytest.mark.parametrize("split,nb", TILES)
+def test_layer_cols_per_item(env, split, nb, knob_env):
     """A launch over part of the columns (the windowed decode's form: middle items [q0, q0 + nq),
     item 0 from ext_l earlier, the last item to ext_r later, tile shape of the full width) writes
     exactly those columns of each item, bit-identical to the full launch, and nothing else: conv
     and both convT layers, an MRF K = 11 conv at dilation 5, conv_post; batches 1, 2 and 3; every
-    tile shape (rb, split 0: the launcher's choice)."""
+    tile shape (two column blocks only where a launch's window allows them: not K = 11 at dilation 5)."""
     ctx, model, ws, bs = env
-    say(f"layer columns rb={rb} split={split}")
-    if rb:
-        knob_env.setenv("PTK_CONV_RB", str(rb))
-        knob_env.setenv("PTK_CONV_SPLIT", str(split))
+    say(f"layer columns split={split} nb={nb}")
+    _force_tile(knob_env, split, nb)
     lib = ctx.lib
-    rng = np.random.default_rng(rb * 10 + split)
+    rng = np.random.default_rng(10 * split + nb)
     for layer, T, off, nq, el, er in LAYER_COLS:
         g = synth.dec_layer(layer)
         cin, cout4 = g["cin"], (g["cout"] + 3) // 4 * 4
@@ -321,20 +329,17 @@ def test_layer_cols_per_item(env, rb, split, knob_env):
             dx.free(); dfull.free(); dy.free()
 
 
-@pytest.mark.parametrize("rb,split", [(16, 1), (16, 2), (16, 4), (16, 8), (32, 1), (32, 2), (32, 4),
-                                      (32, 8)])
-def test_tile_shapes_vs_oracle(env, rb, split, knob_env):
-    """Every tile shape the launcher can pick (16- or 32-row tiles, channel split 1 / 2 / 4, and 8
-    on the single-problem launches; forced through PTK_CONV_RB / PTK_CONV_SPLIT) against the
-    oracle: a conv with a LeakyReLU epilogue,
+@pytest.mark.parametrize("split,nb", TILES)
+def test_tile_shapes_vs_oracle(env, split, nb, knob_env):
+    """Every tile shape the launcher can pick (channel split 2 / 4, column blocks per wave 1 / 2;
+    forced through PTK_CONV_SPLIT / PTK_CONV_NB) against the oracle: a conv with a LeakyReLU epilogue,
     both convT phase forms (input LeakyReLU, C4 = 256 and 128), the 72-row conv_post whose last
     row block is partial, an MRF stack (grouped K 3 / 7 / 11, residual adds, branch sums) and a
     whole decode."""
     ctx, model, ws, bs = env
-    say(f"tile shape rb={rb} split={split}")
-    knob_env.setenv("PTK_CONV_RB", str(rb))
-    knob_env.setenv("PTK_CONV_SPLIT", str(split))
-    rng = np.random.default_rng(40 + rb + split)
+    say(f"tile shape split={split} nb={nb}")
+    _force_tile(knob_env, split, nb)
+    rng = np.random.default_rng(40 + 10 * split + nb)
     cases = [(0, 226, 0.0, 0.1), (1, 61, 0.1, 0.0), (20, 97, 0.1, 0.0), (39, 203, 0.0, 0.0)]
     for layer, T, in_a, epi_a in cases:
         g = synth.dec_layer(layer)
@@ -367,51 +372,59 @@ def test_tile_shapes_vs_oracle(env, rb, split, knob_env):
     assert np_ref.sndr(wav, ref) >= 60.0
 
 
-@pytest.mark.parametrize("rb,split", [(0, 0), (16, 4), (16, 8), (32, 8)])
-def test_general_epilogue_matches_fast(env, rb, split, knob_env):
+@pytest.mark.parametrize("split,nb", TILES)
+def test_general_epilogue_matches_fast(env, split, nb, knob_env):
     """The per-element epilogue (every block forced onto it with PTK_CONV_FAST=0) writes the fast
     epilogue's bits: a conv with a LeakyReLU epilogue, both convTs (the decoder's rows
-    interleaved by phase, whose fast path stores sample pairs), conv_post with its partial row
-    block, an MRF stack (residual adds) and whole decodes at batch 2 (the convTs' LeakyReLU
-    copies, the branch averages); on the launcher's tiles and forced 16-row / 8-way ones."""
+    interleaved by phase), conv_post with its partial row block, an MRF stack (residual adds) and whole
+    decodes at batch 2 (the convTs' LeakyReLU copies, the branch averages); on every tile shape."""
     ctx, model, ws, bs = env
-    say(f"general vs fast epilogue rb={rb} split={split}")
-    if rb:
-        knob_env.setenv("PTK_CONV_RB", str(rb))
-        knob_env.setenv("PTK_CONV_SPLIT", str(split))
-    lib = ctx.lib
-
-    def run_all():
-        outs = []
-        for layer, T, in_a, epi_a in [(0, 226, 0.0, 0.1), (1, 61, 0.1, 0.0), (20, 97, 0.1, 0.0),
-                                      (39, 203, 0.0, 0.0)]:
-            g = synth.dec_layer(layer)
-            x = np.random.default_rng(layer).standard_normal((g["cin"], T)).astype(np.float32)
-            c4 = (g["cout"] + 3) // 4 * 4
-            tout = 4 * T if g.get("convT") else T
-            dx, dy = dev_of(ctx, x), pkg.DevBuf(c4 * tout)
-            assert lib.ptd_layer(ctx.ptr, model.ptr, layer, dx.ptr, T, 1, dy.ptr, in_a, epi_a) == 0
-            outs.append(dy.download(ctx))
-            dx.free(); dy.free()
-        x = np.random.default_rng(3).standard_normal((128, 300)).astype(np.float32)
-        dx, dy = dev_of(ctx, x), pkg.DevBuf(128 * 300)
-        assert lib.ptd_mrf(ctx.ptr, model.ptr, 1, dx.ptr, 300, 0.1, dy.ptr) == 0
-        outs.append(dy.download(ctx))
-        dx.free(); dy.free()
-        for T in (3, 45):
-            z = np.stack([synth.latent(T, 600 + T), synth.latent(T, 700 + T)])
-            dz, dw = dev_of(ctx, z), pkg.DevBuf(2 * 256 * T)
-            assert lib.ptd_decode(ctx.ptr, model.ptr, dz.ptr, T, 2, dw.ptr) == 0
-            outs.append(dw.download(ctx))
-            dz.free(); dw.free()
-        return outs
-
-    fast = run_all()
+    say(f"general vs fast epilogue split={split} nb={nb}")
+    _force_tile(knob_env, split, nb)
+    fast = _run_convs(env)
     knob_env.setenv("PTK_CONV_FAST", "0")
-    general = run_all()
-    knob_env.delenv("PTK_CONV_FAST")
+    general = _run_convs(env)
     for i, (a, b) in enumerate(zip(fast, general)):
         assert np.array_equal(a, b), i
+
+
+@pytest.mark.parametrize("split", [2, 4])
+def test_column_blocks_change_no_bit(env, split, knob_env):
+    """One or two column blocks per wave: the same bits (S alone fixes the order of a sum)."""
+    say(f"column blocks at split={split}")
+    _force_tile(knob_env, split, 1)
+    one = _run_convs(env)
+    knob_env.setenv("PTK_CONV_NB", "2")
+    for i, (a, b) in enumerate(zip(one, _run_convs(env))):
+        assert np.array_equal(a, b), i
+
+
+def _run_convs(env):
+    ctx, model, ws, bs = env
+    lib = ctx.lib
+    outs = []
+    for layer, T, in_a, epi_a in [(0, 226, 0.0, 0.1), (1, 61, 0.1, 0.0), (20, 97, 0.1, 0.0),
+                                  (39, 203, 0.0, 0.0)]:
+        g = synth.dec_layer(layer)
+        x = np.random.default_rng(layer).standard_normal((g["cin"], T)).astype(np.float32)
+        c4 = (g["cout"] + 3) // 4 * 4
+        tout = 4 * T if g.get("convT") else T
+        dx, dy = dev_of(ctx, x), pkg.DevBuf(c4 * tout)
+        assert lib.ptd_layer(ctx.ptr, model.ptr, layer, dx.ptr, T, 1, dy.ptr, in_a, epi_a) == 0
+        outs.append(dy.download(ctx))
+        dx.free(); dy.free()
+    x = np.random.default_rng(3).standard_normal((128, 300)).astype(np.float32)
+    dx, dy = dev_of(ctx, x), pkg.DevBuf(128 * 300)
+    assert lib.ptd_mrf(ctx.ptr, model.ptr, 1, dx.ptr, 300, 0.1, dy.ptr) == 0
+    outs.append(dy.download(ctx))
+    dx.free(); dy.free()
+    for T in (3, 45):
+        z = np.stack([synth.latent(T, 600 + T), synth.latent(T, 700 + T)])
+        dz, dw = dev_of(ctx, z), pkg.DevBuf(2 * 256 * T)
+        assert lib.ptd_decode(ctx.ptr, model.ptr, dz.ptr, T, 2, dw.ptr) == 0
+        outs.append(dw.download(ctx))
+        dz.free(); dw.free()
+    return outs
 
 
 def _oracle_windows(ws, bs, z, win, ctx_):
@@ -521,8 +534,8 @@ def test_window_columns_change_no_sample(env, T, win, cx, knob_env):
 @pytest.mark.parametrize("T,win,cx", [(1500, 96, 16), (400, 64, 12), (48, 48, 16)])
 def test_windowed_decode_judges_no_unread_column(env, T, win, cx):
     """A launch over part of the columns neither stages nor judges the ones beside them, which
-    nobody wrote: with the arena full of NaN a windowed decode sends no workgroup to look at its
-    columns one by one (ordinary latents: a handful of values at most may call for it)."""
+    nobody wrote: with the arena full of NaN a windowed decode sends no workgroup on a
+    second pass over them (ordinary latents: a handful of values at most may call for it)."""
     ctx, model, ws, bs = env
     say(f"windowed decode's unread columns T={T} win={win} ctx={cx}")
     z = synth.latent(T, 4300 + T)
@@ -532,7 +545,7 @@ def test_windowed_decode_judges_no_unread_column(env, T, win, cx):
     assert ctx.lib.ptd_debug_conv_stats(n0) == 0
     assert ctx.lib.ptd_decode_windows(ctx.ptr, model.ptr, dz.ptr, T, win, cx, dw.ptr) == 0
     assert ctx.lib.ptd_debug_conv_stats(n1) == 0
-    say(f"  looked at columns: {n1[0] - n0[0]} workgroups, second pass: {n1[1] - n0[1]}")
+    say(f"  left outputs: {n1[0] - n0[0]} workgroups, second pass: {n1[1] - n0[1]}")
     # the decode's conv launches have thousands of workgroups; unread columns alarmed hundreds
     assert n1[0] - n0[0] <= 16 and n1[1] == n0[1]
     dz.free(); dw.free()
