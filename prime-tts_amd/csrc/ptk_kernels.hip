@@ -1251,7 +1251,10 @@ conv_mfma_kernel(const ConvGroup g) {
   // in bounds without a branch (a lane whose column does not exist stores nothing).  The chain runs
   // op by op over a lane's values, one branch per op.  A convT block with its rows interleaved by
   // phase (phase_il) holds 8 whole channels.
-  if ((pi.flags & PROB_FAST) && (one_phase || phase_il) && mb * 32 + 32 <= pi.M) {
+  // A partial block (the rows of a conv behind its last output) stores the groups that exist; its
+  // bias reads 0 past the end, its scale is there for every row, a residual would not be.
+  const bool part_block = mb * 32 + 32 > pi.M;
+  if ((pi.flags & PROB_FAST) && (one_phase || phase_il) && (!part_block || (addt < 0 && pi.M == pi.C4 && pi.M % 4 == 0))) {
     const ConvEpi ep = g.ep[p];
     // first channel of the block
     const long long row0 = phase_il ? (long long) mb * 8 : (long long) mb * 32 - (long long) r_tile * ep.C4;
@@ -1271,6 +1274,7 @@ conv_mfma_kernel(const ConvGroup g) {
     // wave-uniform part of the row of value i (the lane part is 4 * half)
     auto urow = [&](int i) { return 8 * ((v0 + i) >> 2) + ((v0 + i) & 3); };
     const int qend32 = ep.qend + (last_item ? ep.ext_r : 0);
+    const int rows = pi.M - mb * 32 - 4 * half;
     float rv[NB][NMAX];
     if (addt >= 0) {
 #pragma unroll
@@ -1340,7 +1344,7 @@ conv_mfma_kernel(const ConvGroup g) {
         const int vg = v0 + gg * GRP;
         const int cg = phase_il ? col + (vg >> 2) : col;
         const int rg = phase_il ? (vg & 3) : urow(gg * GRP);   // uniform part of the group's first row
-        if (!(oq && cg >= 0 && cg < ep.lout && (left >> (nb * NG + gg) & 1) == pass)) continue;
+        if (!(oq && cg >= 0 && cg < ep.lout && 8 * (vg >> 2) < rows && (left >> (nb * NG + gg) & 1) == pass)) continue;
         const unsigned vo = (unsigned) (4 * half * ldy32 + cg) * 4u;
 #pragma unroll
         for (int i = 0; i < GRP; i++) {
@@ -1367,7 +1371,8 @@ conv_mfma_kernel(const ConvGroup g) {
       }
     }
   } else {
-  // General path (partial row blocks, convT phases that straddle a block, large tensors): per
+  // General path (partial row blocks of a convT or with a residual, convT phases that straddle a
+  // block, large tensors): per
   // element
   const int M = d.M, C4 = d.C4, ys = d.ys, ypad = d.ypad, nepi = d.nepi;
   const long long Lout = d.Lout, ldy = d.ldy;
