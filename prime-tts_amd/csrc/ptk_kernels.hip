@@ -1515,24 +1515,32 @@ extern "C" void ptk_knobs_reload(void) {
 
 // Tile shape: the channel split S in {2, 4} (PTK_CONV_SPLIT overrides) and the column blocks per
 // wave NB in {1, 2} (PTK_CONV_NB).
-// Measured: S = 2 against 4 at C 128, T 3616, batch 8 159-165 against 175-195 us, at C 256, T 904 37
-// against 30 us; NB = 2 against 1 for the MRF-256 group at T 904 30 against 33 us, at T 252 22.8
-// against 17.8 us, ups.0 at T 226 12.5 against 10.3 us, conv_pre at batch 8 13 against 16.6 us.
 // S fixes the order in which a block's partial sums are added, so it is chosen from one batch item's
 // grid (of nq_shape columns when the launch covers a sub-range): a batched item's result is
-// bit-identical to the same item alone.  NB changes no bit and is chosen from the whole launch.
+// bit-identical to the same item alone.  Measured: S = 2 against 4 at C 128, T 3616, batch 8 159-165
+// against 175-195 us, at C 256, T 904 37 against 30 us.
+// NB changes no bit and is chosen from the whole launch.  Up to a few workgroups per CU a launch takes
+// as long as its fullest CU, and a workgroup of two column blocks 1.2 to 1.4 times one of one block:
+// two are worth it where they take a round of 256 workgroups less, and from 512 on, where every CU has
+// several either way.  One against two blocks, us, S = 4: K 3, C 256, 232 / 120 workgroups 6.6 / 8.2,
+// 408 / 208 9.0 / 8.3, 504 / 264 9.2 / 10.9, 512 / 256 9.2 / 8.3; K 11, C 128, 372 / 192 8.8 / 8.1;
+// ups.0, 256 / 128 10.1 / 11.9, 576 / 288 19.5 / 18.5; conv_post 342 / 171 7.1 / 6.8, 744 / 384
+// 9.7 / 9.8.  Grouped launches, whose problems are of different weight, from 200 (per depth of an
+// MRF-256 stack, 384 / 192 10.8 / 11.8, 696 / 360 16.0 / 14.5).
 static void choose_tiles(const ptk_conv_desc *const *ds, int n, int *S_out, int *nb_out) {
   const int env_s = knob(KN_CONV_SPLIT), env_nb = knob(KN_CONV_NB);
   bool nb2_ok = true;
-  long long wgs = 0, item = 0;
+  long long wgs1 = 0, wgs = 0, item = 0;
   for (int i = 0; i < n; i++) {
     const ptk_conv_desc *d = ds[i];
     if (conv_window(d, 2) > 32 * CONV_NU_MAX) nb2_ok = false;
     const long long mt = (d->M + 31) / 32, nq = d->nq_shape > 0 ? d->nq_shape : d->nq;
+    wgs1 += d->batch * mt * ((d->nq + 31) / 32);
     wgs += d->batch * mt * ((d->nq + 63) / 64);
     item += mt * ((nq + 63) / 64);
   }
-  *nb_out = nb2_ok && (env_nb == 2 || (env_nb != 1 && wgs >= 200)) ? 2 : 1;
+  const bool two = n > 1 ? wgs >= 200 : wgs >= 512 || (wgs + 255) / 256 < (wgs1 + 255) / 256;
+  *nb_out = nb2_ok && (env_nb == 2 || (env_nb != 1 && two)) ? 2 : 1;
   *S_out = env_s == 2 || env_s == 4 ? env_s : item >= 640 ? 2 : 4;
 }
 
