@@ -154,7 +154,6 @@ int ptk_relayout(float *dst, const float *wp, int M, int K, int cin, void *s);
 /* the same with a stride-4 convT's rows interleaved by phase: il = its rows per phase C4, a multiple
    of 8, M = 4 * il */
 int ptk_relayout_il(float *dst, const float *wp, int M, int K, int cin, int il, void *s);
-int ptk_relayout16_il(float *dst, const float *wp, int M, int K, int cin, int il, void *s);
 /* fp16 -> fp32 expansion of n items (bit-exact: subnormals keep their value, inf / NaN keep sign
  * and payload, nothing is quieted) */
 int ptk_h2f(float *dst, const uint16_t *src, int64_t n, void *s);

@@ -573,10 +573,6 @@ extern "C" int ptk_relayout_il(float *dst, const float *wp, int M, int K, int ci
 extern "C" int ptk_relayout(float *dst, const float *wp, int M, int K, int cin, void *s) {
   return ptk_relayout_il(dst, wp, M, K, cin, 0, s);
 }
-// (one layout serves every tile; the name stays for callers that have it)
-extern "C" int ptk_relayout16_il(float *dst, const float *wp, int M, int K, int cin, int il, void *s) {
-  return ptk_relayout_il(dst, wp, M, K, cin, il, s);
-}
 
 // ------------------------------------------------------------------------------ fp16 expansion
 // binary16 -> binary32 by its bit fields.  Every binary16 value is exact in binary32: normals
