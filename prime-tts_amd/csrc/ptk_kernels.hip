@@ -422,14 +422,14 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsign
   h = __builtin_bit_cast(unsigned, h2{ha, hb});
   l = f16_pair(__builtin_fmaf((float) ha, -1.0f, a), __builtin_fmaf((float) hb, -1.0f, b));
 }
-// and of a pair of inputs, which it scales (exact: powers of two, and the fma's result is)
+// and of a pair of inputs, which it scales by 2^CONV_XS (exact: powers of two, and the fma's result is);
+// written so that each part is one mixed-precision fma of the input times both scales
 __device__ __forceinline__ void split_input(float a, float b, unsigned &h, unsigned &l) {
-  constexpr float X = (float) (1 << CONV_XS);
-  const _Float16 ha = (_Float16) (a * X), hb = (_Float16) (b * X);
+  const float a2 = a * ((float) (1 << CONV_XS) * CONV_LS), b2 = b * ((float) (1 << CONV_XS) * CONV_LS);
+  const _Float16 ha = (_Float16) __builtin_fmaf(a2, 1.0f / CONV_LS, 0.0f), hb = (_Float16) __builtin_fmaf(b2, 1.0f / CONV_LS, 0.0f);
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
   h = __builtin_bit_cast(unsigned, h2{ha, hb});
-  l = f16_pair(__builtin_fmaf((float) ha, -CONV_LS, a * (X * CONV_LS)),
-               __builtin_fmaf((float) hb, -CONV_LS, b * (X * CONV_LS)));
+  l = f16_pair(__builtin_fmaf((float) ha, -CONV_LS, a2), __builtin_fmaf((float) hb, -CONV_LS, b2));
 }
 
 // Split planes: an activation tensor [C][T] already in two parts, scaled by 2^CONV_XS, as
