@@ -1168,24 +1168,29 @@ conv_mfma_kernel(const ConvGroup g) {
     }
     const int qend = pi.qend + (last_item ? pi.ext_r : 0);
     unsigned low = 0;   // bit 4 * nb + (v >> 2): rows 8 * (v >> 2) .. + 7 of column block nb
+    unsigned long long used[NB], any = 0;
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
-      const unsigned long long used = __ballot(q0 + 32 * nb + l32 < qend);
+      float m = __builtin_inff();
 #pragma unroll
-      for (int v = 0; v < 16; v += 4) {
-        const float m = min_mag(min_mag(__builtin_inff(), acc[nb][v], acc[nb][v + 1]), acc[nb][v + 2], acc[nb][v + 3]);
-        low |= (__ballot(!(m >= thr_b)) & used) != 0 ? 1u << (4 * nb + v / 4) : 0u;
-      }
+      for (int v = 0; v < 16; v += 2) m = min_mag(m, acc[nb][v], acc[nb][v + 1]);
+      used[nb] = __ballot(q0 + 32 * nb + l32 < qend);
+      any |= __ballot(!(m >= thr_b)) & used[nb];
     }
-    const int rows = pi.M - mb * 32;   // (the padding rows behind them are all zero)
-    low &= rows >= 32 ? 0xffu : 0x11u * ((1u << ((rows + 7) >> 3)) - 1);
-    if (low != 0) {   // a NaN makes the workgroup judge whatever the other waves have
-      float m = 0.0f;
+    if (any != 0) {   // (a few in a hundred of a large launch's waves)
+      float all = 0.0f;
 #pragma unroll
       for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-        for (int v = 0; v < 16; v += 2) m = min_mag(m, acc[nb][v], acc[nb][v + 1]);
-      if (__ballot(m != m) != 0) low |= 0x100;
+        for (int v = 0; v < 16; v += 4) {
+          const float m = min_mag(min_mag(__builtin_inff(), acc[nb][v], acc[nb][v + 1]), acc[nb][v + 2], acc[nb][v + 3]);
+          all = min_mag(all, m, m);
+          low |= (__ballot(!(m >= thr_b)) & used[nb]) != 0 ? 1u << (4 * nb + v / 4) : 0u;
+        }
+      const int rows = pi.M - mb * 32;   // (the padding rows behind them are all zero)
+      low &= rows >= 32 ? 0xffu : 0x11u * ((1u << ((rows + 7) >> 3)) - 1);
+      // a NaN makes the workgroup judge whatever the other waves have
+      if (__ballot(all != all) != 0) low |= 0x100;
     }
     if (lane == 0) flags[w] = nch > 0 ? (int) low : 0xff;   // (a wave without channels has no say)
     if (threadIdx.x == 0) flags[4] = flags[5] = 0;
