@@ -559,8 +559,11 @@ int ptd_tail(pt_ctx *c, const ptd_model *m, const float *p, int64_t L, int batch
 size_t ptd_decode_arena_bytes(int64_t T, int batch) {
   const size_t f = sizeof(float) * (size_t) batch;
   const int64_t T1 = 4 * T, T2 = 16 * T, L = T2 + 1;
+  /* An upper bound that requests were sized and refused by since the copies were fp32: decode_impl
+   * holds hS too, but gives ups.1's and conv_post's inputs and MRF-128's temporaries the same
+   * place, which leaves about a tenth unused. */
   size_t s = 0;
-  s += al256(f * 512 * T) + 2 * al256(f * 256 * T1) + 3 * al256(f * 256 * T1);   /* h, x0, x0L, o[] */
+  s += al256(f * 512 * T) + 2 * al256(f * 256 * T1) + 3 * al256(f * 256 * T1);   /* h, x0, x0S, o[] */
   size_t mrf0 = 9 * al256(f * 256 * T1);
   size_t late = 2 * al256(f * 128 * T2) + 3 * al256(f * 128 * T2) + 9 * al256(f * 128 * T2) +
                 al256(f * 72 * L) + al256(f * 256 * T1) + al256(f * 128 * T2);

@@ -397,7 +397,8 @@ extern "C" int ptk_graph_destroy(void *exec) {
 #define CONV_LA2 2
 #endif
 // The inputs' scale, 2^CONV_XS: up to 2^12 an input fits its fp16 parts, and outputs of N(0, s) inputs
-// keep to the first pass down to about s = 2^-8 (a larger scale moves both ends down).
+// keep to the first pass down to about s = 2^-6, below that all but a few workgroups do (a larger scale
+// moves both ends down).
 #define CONV_XS 4
 #define CONV_LS 2048.0f    // the scale of the inputs' lo
 
@@ -780,11 +781,14 @@ __device__ unsigned long long conv_stat[2];
 // output comes from depends on its own receptive field and the four rows' weights, not on the tile
 // or batch it is computed in.  Outputs that see nothing but zeros are left too, and skip that pass.
 //
-// Bound by the matrix cores on large launches (552 TFLOP/s of fp32 products at the rate the card
-// sustains, 150 on the fp32 matrix cores), by the way in and out of a workgroup on small ones.
-// Against the fp32-MFMA kernel it replaced: MRF-256 stack at T 904 149 -> 82 us, MRF-128 at T 3616
-// 154 -> 98 us, conv_pre at T 226 6.35 -> 5.6 us, ups.0 11.4 -> 9.5 us, a T 226 decode 345 -> 221 us
-// and eight in a batch 2141 -> 987 us; errors against 64 bits 0.36-0.90 of what they were on N(0, 1).
+// Against a floor of 552 TFLOP/s of fp32 products (the fp16 rate the card sustains; 150 on the fp32
+// matrix cores) it is bound by the way in and out of a workgroup (first loads, partial sums, stores),
+// at batch 8 by operand loads as well: the matrix cores are 13-17 % busy in a T 226 decode's MRF
+// launches, 37-45 % in eight of them (rocprofv3).  Against the fp32-MFMA kernel it replaced, us: MRF-256
+// stack at T 904 149 -> 89, MRF-128 at T 3616 154 -> 109, conv_pre at T 226 6.3 -> 5.8, ups.0 11.4 ->
+// 9.7, a T 226 decode 345 -> 241 and eight in a batch 2167 -> 1030; errors against 64 bits 0.36-0.90 of
+// what they were on N(0, 1).  Inputs past 2^12, whose outputs take both passes: MRF-256 320-330, a T 226
+// decode 810-880.
 //
 // KT: the taps the straight-line bodies are built for (11: K = 11, 7 and 3; 4: K = 4, the convT
 // phase form); any other K goes through a rolled loop.  IN: input transform (PTK_IN_*).
@@ -2702,7 +2706,7 @@ extern "C" int ptk_mfma_probe(const float *a, const float *b, float *d, void *s)
 }
 
 // 16x16x4: lane l holds A[l % 16][l / 16] and B[l / 16][l % 16]; value r of its result is
-// D[4*(l / 16) + r][l % 16], the layout the 16-row conv tiles assume
+// D[4*(l / 16) + r][l % 16], the layout the tail's products assume
 __global__ void mfma16_probe_kernel(const float *a, const float *b, float *d) {
   const int lane = threadIdx.x;
   f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};

@@ -97,7 +97,7 @@ def test_mfma_lane_layout(ctx):
 
 def test_mfma16_lane_layout(ctx):
     """The same for the fp32 16x16x4 builtin: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and
-    result rows 4*(l / 16) + r of column l % 16 (the layout of the 16-row conv tiles)."""
+    result rows 4*(l / 16) + r of column l % 16 (the layout of the tail's products)."""
     say("mfma16 probe")
     rng = np.random.default_rng(1)
     a = rng.standard_normal((16, 4)).astype(np.float32)
