@@ -260,3 +260,17 @@ def test_ordinary_inputs_and_silence_stay_on_the_first_pass(ctx):
     assert _stats(ctx)[1] > n2[1]
     want = np.float64(W[:, 17, ::-1]) * np.float64(x[0, 17, 200])
     assert np.all(np.abs(y[0, :, 197:204] - want) <= 2.0 ** -23 * np.abs(want))
+
+
+@pytest.mark.parametrize("cout", [30, 37, 62, 70, 97])
+@pytest.mark.parametrize("nb", [1, 2])
+def test_rows_of_a_partial_block(ctx, cout, nb, knob_env):
+    """Outputs that do not fill their last block of 32 rows, nor its last group of four: bias and
+    LeakyReLU of the ones that exist, and nothing behind them is written over (batch 2: the rows of the
+    next item follow)."""
+    knob_env.setenv("PTK_CONV_NB", str(nb))
+    rng, x, W, b = case(48, cout, 7, 133, seed=11, B=2)
+    y = gpu_conv(ctx, x, synth.pack_conv(W), b, cout, 7, 1, 3, 1)
+    ref, mag = conv64(x, W, b, 3, 1, 1)
+    bound = (48 * 7 * 1.5 + 9) * 2.0 ** -24 * (mag + np.abs(b.astype(np.float64))[:, None])
+    assert np.all(np.abs(y[:, :cout] - ref) <= bound)
