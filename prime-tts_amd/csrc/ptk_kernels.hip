@@ -370,7 +370,7 @@ extern "C" int ptk_graph_destroy(void *exec) {
 // threshold per row that relayout_kernel makes.
 //
 // Packed [M/4][K][cin][4] (the reference's conv layout; a convT's phase rows are just more rows)
-// -> three parts, one after the other (Mp: M rounded up to 32, cinp: cin rounded up to 16; padding
+// -> these parts, one after the other (Mp: M rounded up to 32, cinp: cin rounded up to 16; padding
 // rows and channels are zero):
 //   fp16 [Mp/32][cinp/16][K][2][64][8]: for a row block mb, a chunk of 16 input channels and a tap k,
 //     lane l = 32*h + r of a wave holds, of hi and of lo, the eight scaled values
